@@ -337,11 +337,19 @@ void FFAExecutor::init_level(const float* ts_e, const float* ts_v, void* out, vo
     }
     if (!m_lossy) {
         const double t_ref = m_freq_only ? 0.0 : m_plan.tsegments()[0] / 2.0;
-        kern::brute_fold_fourier(ts_e, ts_v, nseg, static_cast<uint32_t>(m_plan.segment_lens()[0]),
-                                 m_bf_freqs.as<double>(),
-                                 static_cast<uint32_t>(m_plan.param_counts()[0].back()),
-                                 static_cast<uint32_t>(nbins), m_plan.config().get_tsamp(),
-                                 t_ref, static_cast<float2*>(out), s, m_dft_split);
+        const auto seglen  = static_cast<uint32_t>(m_plan.segment_lens()[0]);
+        const auto nfreqs  = static_cast<uint32_t>(m_plan.param_counts()[0].back());
+        const auto nb      = static_cast<uint32_t>(nbins);
+        if (!m_dft_split && kern::spectra_fold_better(seglen, nfreqs)) {
+            m_ws->spectra.reserve(kern::spectra_bytes(nseg, seglen));
+            kern::brute_fold_spectra(ts_e, ts_v, nseg, seglen, m_bf_freqs.as<double>(), nfreqs, nb,
+                                     m_plan.config().get_tsamp(), t_ref,
+                                     static_cast<float2*>(out), m_ws->spectra.get(), s);
+        } else {
+            kern::brute_fold_fourier(ts_e, ts_v, nseg, seglen, m_bf_freqs.as<double>(), nfreqs, nb,
+                                     m_plan.config().get_tsamp(), t_ref,
+                                     static_cast<float2*>(out), s, m_dft_split);
+        }
         check_launch("Fourier brute fold launch");
         m_timer.stop(bslot, s);
         return;
@@ -819,12 +827,21 @@ void brute_fold_fourier_device(const float* ts_e, const float* ts_v, SizeType ns
     hip_check(hipMemcpyAsync(d_freqs.get(), freqs.data(), freqs.size() * sizeof(double),
                              hipMemcpyHostToDevice, s),
               "copy frequencies");
-    kern::brute_fold_fourier(ts_e, ts_v, nsamps / segment_len,
-                             static_cast<uint32_t>(segment_len), d_freqs.as<double>(),
-                             static_cast<uint32_t>(freqs.size()), static_cast<uint32_t>(nbins),
-                             tsamp, t_ref, fold, s);
+    const auto seglen = static_cast<uint32_t>(segment_len);
+    const auto nfreqs = static_cast<uint32_t>(freqs.size());
+    const auto nb     = static_cast<uint32_t>(nbins);
+    const SizeType ns = nsamps / segment_len;
+    DeviceBuffer d_spec;
+    if (kern::spectra_fold_better(seglen, nfreqs)) {
+        d_spec.reserve(kern::spectra_bytes(ns, seglen));
+        kern::brute_fold_spectra(ts_e, ts_v, ns, seglen, d_freqs.as<double>(), nfreqs, nb, tsamp,
+                                 t_ref, fold, d_spec.get(), s);
+    } else {
+        kern::brute_fold_fourier(ts_e, ts_v, ns, seglen, d_freqs.as<double>(), nfreqs, nb, tsamp,
+                                 t_ref, fold, s);
+    }
     check_launch("Fourier brute fold launch");
-    // The frequencies are freed on return: finish before releasing them.
+    // The frequencies and spectra are freed on return: finish before that.
     hip_check(hipStreamSynchronize(s), "Fourier brute fold");
 }
 

@@ -64,7 +64,8 @@ private:
 };
 
 /// Device buffers an FFA borrows (workspace.hpp:169-206 FFAWorkspaceCUDA): the
-/// ping-pong partner, the second scores buffer and the shift tables.  FFAs
+/// ping-pong partner, the second scores buffer, the shift tables and the chunk
+/// spectra.  FFAs
 /// that share one run one at a time; each grows the buffers to its plan.
 /// Uses on different streams are ordered: a use on stream s first waits for
 /// an event recorded at the end of the previous use on another stream.
@@ -77,6 +78,7 @@ struct FFAWorkspace {
     DeviceBuffer internal;
     DeviceBuffer result;
     DeviceBuffer coords;
+    DeviceBuffer spectra;  ///< chunk spectra of the Fourier brute fold
 
     /// Before enqueueing work that touches the buffers on `s`.
     void begin_use(hipStream_t s);

@@ -129,6 +129,29 @@ void brute_fold_fourier(const float* ts_e, const float* ts_v, uint64_t nseg, uin
                         const double* freqs_dev, uint32_t nfreqs, uint32_t nbins, double tsamp,
                         double t_ref, float2* fold, hipStream_t s, bool split_bf16 = false);
 
+/// FFT length and number of the chunks a segment of seglen samples is cut into
+/// for its spectra (nufft_device.hpp): power-of-two chunks of 64 to 2048
+/// samples, the last one zero-padded.
+struct SpectraShape {
+    uint32_t m;
+    uint64_t nchunk;
+};
+SpectraShape spectra_shape(uint64_t seglen);
+/// Bytes of the spectra of nseg segments.
+uint64_t spectra_bytes(uint64_t nseg, uint64_t seglen);
+/// Spectra of every chunk of nseg segments of both series.
+void chunk_spectra(const float* ts_e, const float* ts_v, uint64_t nseg, uint64_t seglen,
+                   void* spec, hipStream_t s);
+
+/// Whether brute_fold_spectra is the faster Fourier brute fold.
+bool spectra_fold_better(uint32_t seglen, uint32_t nfreqs);
+/// The Fourier brute fold interpolated from chunk spectra (FP64 FFTs, FP32
+/// values and weights): the same sums as brute_fold_fourier.  spec:
+/// spectra_bytes(nseg, seglen) bytes of workspace, 16-byte aligned.
+void brute_fold_spectra(const float* ts_e, const float* ts_v, uint64_t nseg, uint32_t seglen,
+                        const double* freqs_dev, uint32_t nfreqs, uint32_t nbins, double tsamp,
+                        double t_ref, float2* fold, void* spec, hipStream_t s);
+
 /// Fourier-domain merge of one level (freq-only when coords_freq != nullptr):
 /// phase rotation by the fractional shifts, rows of [2, nbins/2+1] float2.
 void merge_fourier(const float2* in, float2* out, const FFACoord* coords,

@@ -338,8 +338,7 @@ uint64_t spectra_bytes(uint64_t nseg, uint64_t seglen) {
 }
 
 void chunk_spectra(const float* ts_e, const float* ts_v, uint64_t nseg, uint64_t seglen,
-                   void* spec, hipStream_t s) {
-    const auto sh    = spectra_shape(seglen);
+                   const SpectraShape& sh, void* spec, hipStream_t s) {
     const uint64_t n = nseg * sh.nchunk;
     auto* out        = static_cast<float4*>(spec);
     LOKI_REQUIRE(sh.nchunk < (1ULL << 32), "chunk spectra: segment too long");
@@ -372,8 +371,8 @@ void brute_fold_spectra(const float* ts_e, const float* ts_v, uint64_t nseg, uin
     LOKI_REQUIRE(nbins >= 2 && nbins <= 256, "Fourier brute fold: nbins must be in [2, 256]");
     LOKI_REQUIRE(seglen >= 1 && nfreqs >= 1, "Fourier brute fold: empty input");
     LOKI_REQUIRE(nseg >= 1 && 2 * nseg < (1ULL << 31), "Fourier brute fold: too many segments");
-    chunk_spectra(ts_e, ts_v, nseg, seglen, spec, s);
     const auto sh = spectra_shape(seglen);
+    chunk_spectra(ts_e, ts_v, nseg, seglen, sh, spec, s);
     SpecFoldArgs a{};
     a.spec   = static_cast<const float4*>(spec);
     a.fold   = fold;

@@ -139,9 +139,9 @@ struct SpectraShape {
 SpectraShape spectra_shape(uint64_t seglen);
 /// Bytes of the spectra of nseg segments.
 uint64_t spectra_bytes(uint64_t nseg, uint64_t seglen);
-/// Spectra of every chunk of nseg segments of both series.
+/// Spectra of every chunk (sh.m / 2 samples) of nseg segments of both series.
 void chunk_spectra(const float* ts_e, const float* ts_v, uint64_t nseg, uint64_t seglen,
-                   void* spec, hipStream_t s);
+                   const SpectraShape& sh, void* spec, hipStream_t s);
 
 /// Whether brute_fold_spectra is the faster Fourier brute fold.
 bool spectra_fold_better(uint32_t seglen, uint32_t nfreqs);

@@ -41,39 +41,75 @@ __device__ __forceinline__ double spec_inv_window(double x) {
     return fma(p, x, 9.99999999968185782e-01);
 }
 
+/// Even and odd parts of the window about point d, w(s - d) = E_d(s^2) + s O_d(s^2),
+/// as polynomials in s^2 (|s| <= 1/2).
+constexpr int kSpecDeg = 4;
+__device__ constexpr float kSpecEven[kSpecPad + 1][kSpecDeg + 1] = {
+    {4.097066473e-01F, -2.083281511e-01F, 5.045674281e-02F, -7.753501785e-03F, 8.101804419e-04F},
+    {2.448597608e-01F, -1.051982073e-03F, -1.914012523e-02F, 4.811598407e-03F, -6.162238416e-04F},
+    {4.807334798e-02F, 8.947632490e-02F, -1.393384355e-02F, -3.179588528e-04F, 2.512792429e-04F},
+    {2.206964057e-03F, 1.552704906e-02F, 7.236012929e-03F, -9.047692722e-04F, -3.157867915e-05F},
+    {6.603917400e-06F, 2.126500059e-04F, 6.098640552e-04F, 2.880512778e-04F, -1.204746299e-05F}};
+__device__ constexpr float kSpecOdd[kSpecPad + 1][kSpecDeg + 1] = {
+    {0.0F, 0.0F, 0.0F, 0.0F, 0.0F},
+    {2.552360722e-01F, -8.674909089e-02F, 1.350685297e-02F, -1.246088800e-03F, 6.994109597e-05F},
+    {1.088337421e-01F, 2.067225515e-02F, -9.329157141e-03F, 1.229546623e-03F, -8.125434403e-05F},
+    {8.956326233e-03F, 1.452936225e-02F, 1.011406669e-03F, -5.101239540e-04F, 4.719417646e-05F},
+    {5.688209364e-05F, 4.539484141e-04F, 5.305207828e-04F, 7.666968630e-05F, -1.480554840e-05F}};
+
+/// D-th derivative (0, 1 or 2) of a polynomial of degree kSpecDeg at q.
+template <int D>
+__device__ __forceinline__ float spec_poly(const float (&c)[kSpecDeg + 1], float q) {
+    float p = 0.0F;
+#pragma unroll
+    for (int i = kSpecDeg; i >= D; --i) {
+        float k = c[i];
+        if constexpr (D >= 1) {
+            k *= static_cast<float>(i);
+        }
+        if constexpr (D >= 2) {
+            k *= static_cast<float>(i - 1);
+        }
+        p = i == kSpecDeg ? k : fmaf(p, q, k);
+    }
+    return p;
+}
+
 /// Window weights of the points c - 4 .. c + 4 for a position s from point c
-/// (|s| <= 1/2): w(s - d) and w(s + d) share their even and odd parts.
+/// (|s| <= 1/2).
 __device__ __forceinline__ void spec_weights(float s, float (&w)[kSpecTaps]) {
     const float q = s * s;
-    auto poly     = [q](float c0, float c1, float c2, float c3, float c4) {
-        return fmaf(fmaf(fmaf(fmaf(c4, q, c3), q, c2), q, c1), q, c0);
-    };
-    w[4] = poly(4.097066473e-01F, -2.083281511e-01F, 5.045674281e-02F, -7.753501785e-03F,
-                8.101804419e-04F);
-    auto pair = [&](int d, float e, float o) {
-        w[4 + d] = fmaf(s, o, e);
-        w[4 - d] = fmaf(-s, o, e);
-    };
-    pair(1,
-         poly(2.448597608e-01F, -1.051982073e-03F, -1.914012523e-02F, 4.811598407e-03F,
-              -6.162238416e-04F),
-         poly(2.552360722e-01F, -8.674909089e-02F, 1.350685297e-02F, -1.246088800e-03F,
-              6.994109597e-05F));
-    pair(2,
-         poly(4.807334798e-02F, 8.947632490e-02F, -1.393384355e-02F, -3.179588528e-04F,
-              2.512792429e-04F),
-         poly(1.088337421e-01F, 2.067225515e-02F, -9.329157141e-03F, 1.229546623e-03F,
-              -8.125434403e-05F));
-    pair(3,
-         poly(2.206964057e-03F, 1.552704906e-02F, 7.236012929e-03F, -9.047692722e-04F,
-              -3.157867915e-05F),
-         poly(8.956326233e-03F, 1.452936225e-02F, 1.011406669e-03F, -5.101239540e-04F,
-              4.719417646e-05F));
-    pair(4,
-         poly(6.603917400e-06F, 2.126500059e-04F, 6.098640552e-04F, 2.880512778e-04F,
-              -1.204746299e-05F),
-         poly(5.688209364e-05F, 4.539484141e-04F, 5.305207828e-04F, 7.666968630e-05F,
-              -1.480554840e-05F));
+    w[kSpecPad]   = spec_poly<0>(kSpecEven[0], q);
+#pragma unroll
+    for (int d = 1; d <= kSpecPad; ++d) {
+        const float e   = spec_poly<0>(kSpecEven[d], q);
+        const float o   = spec_poly<0>(kSpecOdd[d], q);
+        w[kSpecPad + d] = fmaf(s, o, e);
+        w[kSpecPad - d] = fmaf(-s, o, e);
+    }
+}
+
+/// First (w1) and second (w2) derivatives of the weights in s: they give the
+/// chunk's sums of x_k (k - C) and x_k (k - C)^2 from the same points.
+__device__ __forceinline__ void spec_weights_d(float s, float (&w1)[kSpecTaps],
+                                               float (&w2)[kSpecTaps]) {
+    const float q = s * s;
+    const float t = 2.0F * s;
+#pragma unroll
+    for (int d = 0; d <= kSpecPad; ++d) {
+        const float e1 = spec_poly<1>(kSpecEven[d], q);
+        const float e2 = fmaf(4.0F * q, spec_poly<2>(kSpecEven[d], q), 2.0F * e1);
+        const float o0 = spec_poly<0>(kSpecOdd[d], q);
+        const float o1 = spec_poly<1>(kSpecOdd[d], q);
+        const float a  = fmaf(2.0F * q, o1, o0);
+        const float b  = s * fmaf(4.0F * q, spec_poly<2>(kSpecOdd[d], q), 6.0F * o1);
+        w1[kSpecPad + d] = fmaf(t, e1, a);
+        w2[kSpecPad + d] = e2 + b;
+        if (d > 0) {
+            w1[kSpecPad - d] = fmaf(t, e1, -a);
+            w2[kSpecPad - d] = e2 - b;
+        }
+    }
 }
 
 /// Position of frequency u (turns per sample, u >= 0) on an M-point spectrum:

@@ -126,6 +126,42 @@ def test_ts_v_enters_the_score():
             1e-4 * np.linalg.norm(g_ref / scale) + 2e-3
 
 
+@pytest.mark.parametrize("n,nbins,width", [
+    (1 << 17, 16, 3),             # the shortest series and chunk (128 samples) with spectra
+    ((1 << 18) - 77, 128, 5),     # a short last chunk, more harmonics than a wave
+    ((1 << 19) + 4097, 64, 1),    # chunks of 512
+])
+def test_chunk_spectra_and_sample_loop_candidates(n, nbins, width):
+    """Candidates whose phase is nearly straight over a chunk go through chunk spectra, the
+    others sample by sample, in one call.  The spectra drop the square of at most 2e-4 turns of
+    curvature (8e-7 rad) and round a few FP32 values (~1e-7): 1e-5 bounds both with a margin of
+    ten.  The sample loop keeps its own bound."""
+    from loki_amd import refine
+    from oracle import refine as oref
+
+    torch = _torch()
+    T = n * TSAMP
+    ts_e, ts_v, t_ref = _inject(n, 71, [(61.7, 2.0 / T**2, -5.0 / T**3)], [0.08])
+    scale = np.array(refine.phase_scale(n, TSAMP, t_ref))
+    th = np.array([[61.7, 2.0 / T**2, -5.0 / T**3], [7900.1, -3.0 / T**2, 6.0 / T**3],
+                   [333.3, 0.0, 0.0], [61.7, 4.0e5 / T**2, 0.0], [120.2, 1.0 / T**2, 9.0e6 / T**3]])
+    curved = np.array([False, False, False, True, True])
+    de, dv, dth = _dev(ts_e, ts_v, th)
+    s, st = refine.score_raw(de, dv, dth, TSAMP, t_ref, nbins, width)
+    g = refine.grad_raw(de, dv, dth, st, TSAMP, t_ref, nbins).cpu().numpy()
+    s = s.cpu().numpy().astype(np.float64)
+    for c in range(th.shape[0]):
+        s_ref, g_ref = oref.grad(ts_e, ts_v, TSAMP, t_ref, th[c], nbins, width)
+        err, norm = np.linalg.norm((g[c] - g_ref) / scale), np.linalg.norm(g_ref / scale)
+        print(c, abs(s[c] - s_ref), err / norm)
+        if curved[c]:
+            assert abs(s[c] - s_ref) <= 1e-4 + 1e-5 * abs(s_ref)
+            assert err <= 1e-4 * norm + 2e-3
+        else:
+            assert abs(s[c] - s_ref) <= 1e-5 * (1.0 + abs(s_ref))
+            assert err <= 1e-5 * norm
+
+
 def _gpu_fd(de, dv, th, t_ref, nbins, width, steps):
     """Central differences of the GPU forward, one parameter at a time, for every candidate."""
     from loki_amd import refine

@@ -251,12 +251,16 @@ void FFABatch::build_tasks() {
         std::vector<kern::FoldTask> tasks;
         uint64_t block0 = 0;
         uint32_t max_nbins = 0;
+        uint64_t all_segs  = 0;
+        for (const auto& sr : m_series) {
+            all_segs += (sr.lists.use_runs ? 1U : 0U) == kind ? sr.plan.nsegments()[0] : 0;
+        }
         for (const auto& sr : m_series) {
             const auto& L = sr.lists;
             if ((L.use_runs ? 1U : 0U) != kind) {
                 continue;
             }
-            const uint32_t bps = kern::brute_fold_blocks_per_segment(L);
+            const uint32_t bps = kern::brute_fold_blocks_per_segment(L, all_segs);
             kern::FoldTask t{};
             t.ts_e   = ts_e(static_cast<SizeType>(&sr - m_series.data()));
             t.ts_v   = ts_v(static_cast<SizeType>(&sr - m_series.data()));
@@ -464,7 +468,7 @@ void FFABatch::build_tree(std::vector<uint8_t>& blob, std::vector<SizeType>& off
         t.seglen = L.seglen;
         t.nfreqs = L.nfreqs;
         t.nbins  = L.nbins;
-        t.bps    = kern::brute_fold_blocks_per_segment(L);
+        t.bps    = kern::brute_fold_blocks_per_segment(L, sr.plan.nsegments()[0]);
         ft.push_back(t);
         const auto kind = L.use_runs ? kern::TreeKind::kFoldUnits : kern::TreeKind::kFoldList;
         lds = std::max(lds, kern::tree_lds_bytes(kind, L.nbins, 0, 0));

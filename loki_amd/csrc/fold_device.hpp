@@ -173,114 +173,176 @@ __device__ __forceinline__ uint32_t run_bound(int64_t u, uint32_t n, double tsam
     return lo;
 }
 
-// Long cycles: when a cycle is longer than a chunk, a chunk holds runs of only
-// a short arc of bins, so lanes bound to fixed bins mostly idle.  Here a block
-// owns NF frequencies of one segment with all their bins; their running sums
-// live in LDS, and per chunk the block enumerates the (frequency, bin) units
-// that have samples in the chunk -- for each frequency the bins of the unwrapped
-// range [U(c0), U(c1 - 1)] -- and deals them out to the lanes.  A unit adds all
+// A block owns NF frequencies of one segment with all their bins; their running
+// sums live in LDS, and per chunk of samples the block deals the (frequency,
+// bin) units that have samples in the chunk -- for each frequency the bins of
+// the unwrapped range [U(c0), U(c1 - 1)] -- out to the lanes.  A unit adds all
 // runs of its bin inside the chunk to the bin's running sum in ascending
-// sample order, so every bucket is still the same ordered FP32 sum.
-constexpr int kUnitChunk = 2048;  // samples staged per chunk
-constexpr int kUnitMaxNF = 64;    // frequencies per block (one wave scans their unit counts)
+// sample order, so every bucket is the same ordered FP32 sum as the bucket
+// list's.  The next chunk is on its way into registers, and its units are
+// counted by the last wave, while the units of this one are added.
+//
+// VALU and LDS are about equally busy (24 series of 2^18 to 2^21 samples,
+// 1.3e10 (sample, frequency) pairs, 3.9 ms: 9.3 lane-instructions per pair, two
+// of them the adds, and 2.8 ms of LDS cycles, 43 % of them the runs' bank
+// conflicts).  1024 pairs per block hold four blocks in a CU's LDS; 4096 pairs
+// (three blocks), every boundary by run_bound and the staging unhidden took
+// 5.3 ms.  Chunks of 4096 samples keep more lanes busy where a launch is too
+// small to fill the chip (2^20 samples, 403 frequencies, 0.5-2 Hz: 0.18
+// against 0.20 ms, 0.49 ms before; 2^17 samples 0.03 against 0.21 ms before)
+// and cost a larger one a block per CU (the batch above: 4.6 ms).
+constexpr int kUnitChunk      = 2048;  // samples staged per chunk
+constexpr int kUnitChunkSmall = 4096;  // ... in launches that leave CUs idle
+constexpr uint32_t kUnitPairs = 1024;  // (frequency, bin) pairs per block
+constexpr int kUnitMaxNF      = 64;    // frequencies per block (one wave counts their units)
 
 __host__ __device__ inline uint32_t unit_nf(uint32_t nbins) {
-    const uint32_t nf = 4096U / nbins;  // running sums: nf * nbins * 8 bytes <= 32 KiB
+    const uint32_t nf = kUnitPairs / nbins;
     return nf < 1U ? 1U : (nf > static_cast<uint32_t>(kUnitMaxNF) ? kUnitMaxNF : nf);
 }
 
-__host__ __device__ inline size_t unit_lds_bytes(uint32_t nbins) {
+/// What a block keeps per frequency; the chunk's part twice, in turn.
+struct UnitChunk {
+    double est;        ///< estimated start of bin ulo, from the chunk's first sample
+    int64_t ulo, uhi;  ///< unwrapped bins of the chunk's first and last sample
+    uint32_t cnt, b0;  ///< units in the chunk, bin of the first
+};
+struct UnitFreq {
+    RunGeom g;
+    double sure;  ///< 1/2 less the estimates' error bound (samples)
+    UnitChunk c[2];
+};
+
+__host__ __device__ inline size_t unit_lds_bytes(uint32_t nbins, int chunk = kUnitChunk) {
     const size_t nf = unit_nf(nbins);
-    return kUnitChunk * sizeof(float2) + nf * nbins * sizeof(float2) +
-           nf * (sizeof(RunGeom) + 2 * sizeof(int64_t)) + (kUnitMaxNF + 1) * sizeof(uint32_t);
+    return static_cast<size_t>(chunk) * sizeof(float2) + nf * nbins * sizeof(float2) + nf * sizeof(UnitFreq) +
+           2 * sizeof(uint32_t);
 }
 
-template <typename TO>
+/// First sample of the chunk at or after the beginning of bin ulo + i: the
+/// smallest integer not below est + i A unless that is too close to an
+/// integer to tell (run_bound's margin, so the same value), then run_bound.
+template <int CHUNK>
+__device__ __forceinline__ uint32_t unit_start(const UnitFreq& q, const UnitChunk& c, double i,
+                                               uint32_t c0, uint32_t c1, uint32_t seglen,
+                                               double tsamp, double t_ref, uint32_t nbins) {
+    const double est = fma(i, q.g.A, c.est);
+    const double up  = ceil(est);
+    if (fabs((up - est) - 0.5) < q.sure && est < static_cast<double>(CHUNK)) {
+        const auto k = static_cast<uint32_t>(fmax(up, 0.0));
+        return min(k, c1 - c0);
+    }
+    const uint32_t k =
+        run_bound(c.ulo + static_cast<int64_t>(i), seglen, tsamp, t_ref, q.g, nbins);
+    return min(max(k, c0), c1) - c0;
+}
+
+template <typename TO, int CHUNK = kUnitChunk>
 __device__ __forceinline__ void bf_units_block(uint32_t bid, const float* __restrict__ ts_e,
                                                const float* __restrict__ ts_v, uint32_t seglen,
                                                uint32_t nfreqs, uint32_t nbins,
                                                uint32_t blocks_per_seg,
                                                const double* __restrict__ freqs, double tsamp,
                                                double t_ref, TO* __restrict__ fold, float scale) {
+    constexpr int kPre = CHUNK / kFoldBlock;  // samples a lane stages per chunk
     extern __shared__ __align__(16) unsigned char s_mem[];
-    const uint32_t NF  = unit_nf(nbins);
-    auto* s_ev         = reinterpret_cast<float2*>(s_mem);  // [kUnitChunk], 16-byte aligned
-    auto* acc          = s_ev + kUnitChunk;                   // [NF][nbins]
-    auto* s_geom       = reinterpret_cast<RunGeom*>(acc + NF * nbins);  // [NF]
-    auto* s_ulo        = reinterpret_cast<int64_t*>(s_geom + NF);        // [NF]
-    auto* s_uhi        = s_ulo + NF;                                     // [NF]
-    auto* s_pref       = reinterpret_cast<uint32_t*>(s_uhi + NF);        // [kUnitMaxNF + 1]
+    const uint32_t NF  = (nfreqs + blocks_per_seg - 1) / blocks_per_seg;  // <= unit_nf(nbins)
+    auto* s_ev         = reinterpret_cast<float2*>(s_mem);  // [CHUNK], 16-byte aligned
+    auto* acc          = s_ev + CHUNK;                   // [NF][nbins]
+    auto* fq           = reinterpret_cast<UnitFreq*>(acc + NF * nbins);  // [NF]
+    auto* ncol         = reinterpret_cast<uint32_t*>(fq + NF);  // [2]: most units of a frequency
     const uint64_t seg = bid / blocks_per_seg;
     const uint32_t f0  = (bid % blocks_per_seg) * NF;
+    if (f0 >= nfreqs) {
+        return;
+    }
     const uint32_t nf  = min(NF, nfreqs - f0);
     const float* __restrict__ ge = ts_e + seg * seglen;
     const float* __restrict__ gv = ts_v + seg * seglen;
-    const int64_t nb = nbins;
-    const bool pow2  = (nbins & (nbins - 1U)) == 0;
-    const uint32_t tid = threadIdx.x;
+    const int64_t nb    = nbins;
+    const uint32_t tid  = threadIdx.x;
+    const uint32_t lane = tid % 64;
+    const bool counter  = tid / 64 == kFoldBlock / 64 - 1;  // the counting wave
     for (uint32_t i = tid; i < nf * nbins; i += kFoldBlock) {
         acc[i] = make_float2(0.0F, 0.0F);
     }
-    if (tid < nf) {
-        s_geom[tid] = run_geom(freqs[f0 + tid], seglen, tsamp, t_ref, nbins);
-    }
-    for (uint32_t c0 = 0; c0 < seglen; c0 += kUnitChunk) {
-        const uint32_t c1 = min(c0 + static_cast<uint32_t>(kUnitChunk), seglen);
-        __syncthreads();  // previous chunk's units are done with s_ev and s_pref
-        for (uint32_t k = c0 + tid; k < c1; k += kFoldBlock) {
-            s_ev[k - c0] = make_float2(ge[k], gv[k]);
+    auto count = [&](uint32_t c0, uint32_t turn) {
+        const uint32_t c1 = min(c0 + static_cast<uint32_t>(CHUNK), seglen);
+        uint32_t cnt      = 0;
+        if (lane < nf) {
+            const RunGeom g  = fq[lane].g;
+            const int64_t lo = u_at(c0, tsamp, t_ref, g.f, nbins);
+            const int64_t hi = u_at(c1 - 1, tsamp, t_ref, g.f, nbins);
+            cnt              = hi < lo ? 0U : static_cast<uint32_t>(min(hi - lo + 1, nb));
+            UnitChunk& c     = fq[lane].c[turn];
+            c.est            = (((static_cast<double>(lo) - 0.5) * g.A) + g.B) - c0;
+            c.ulo            = lo;
+            c.uhi            = hi;
+            c.cnt            = cnt;
+            c.b0             = static_cast<uint32_t>(((lo % nb) + nb) % nb);
         }
-        if (tid < kUnitMaxNF) {  // first wave: unit counts and their exclusive scan
-            uint32_t cnt = 0;
-            if (tid < nf) {
-                const double f   = s_geom[tid].f;
-                const int64_t lo = u_at(c0, tsamp, t_ref, f, nbins);
-                const int64_t hi = u_at(c1 - 1, tsamp, t_ref, f, nbins);
-                s_ulo[tid]       = lo;
-                s_uhi[tid]       = hi;
-                cnt = static_cast<uint32_t>(hi - lo + 1 < nb ? hi - lo + 1 : nb);
-            }
-            uint32_t incl = cnt;
-            for (uint32_t o = 1; o < 64; o <<= 1) {
-                const uint32_t y = __shfl_up(incl, o);
-                incl += (tid % 64 >= o) ? y : 0U;
-            }
-            s_pref[tid + 1] = incl;
-            if (tid == 0) {
-                s_pref[0] = 0;
-            }
+        for (int o = 32; o > 0; o >>= 1) {
+            cnt = max(cnt, static_cast<uint32_t>(__shfl_xor(static_cast<int>(cnt), o)));
+        }
+        if (lane == 0) {
+            ncol[turn] = cnt;
+        }
+    };
+    float pe[kPre], pv[kPre];
+    auto fetch = [&](uint32_t c0) {
+#pragma unroll
+        for (int i = 0; i < kPre; ++i) {
+            const uint32_t k = c0 + tid + i * kFoldBlock;
+            pe[i]            = k < seglen ? ge[k] : 0.0F;
+            pv[i]            = k < seglen ? gv[k] : 0.0F;
+        }
+    };
+    fetch(0);
+    if (counter) {
+        if (lane < nf) {
+            const RunGeom g = run_geom(freqs[f0 + lane], seglen, tsamp, t_ref, nbins);
+            fq[lane].g      = g;
+            fq[lane].sure   = 0.5 - ((4.0 * g.eta_len) + 1e-9 +
+                                   32.0 * 0x1p-53 * (static_cast<double>(seglen) + 2.0 * fabs(g.B)));
+        }
+        count(0, 0);
+    }
+    uint32_t turn = 0;
+    for (uint32_t c0 = 0; c0 < seglen; c0 += CHUNK, turn ^= 1U) {
+        const uint32_t c1 = min(c0 + static_cast<uint32_t>(CHUNK), seglen);
+        __syncthreads();  // the previous chunk's units are done with s_ev, this one's counted
+#pragma unroll
+        for (int i = 0; i < kPre; ++i) {
+            s_ev[tid + i * kFoldBlock] = make_float2(pe[i], pv[i]);
         }
         __syncthreads();
-        const uint32_t total = s_pref[nf];
-        uint32_t fi = 0;  // units are ordered by frequency and t only grows
-        for (uint32_t t = tid; t < total; t += kFoldBlock) {
-            uint32_t lo = fi, hi = nf;  // largest fi with s_pref[fi] <= t
-            while (hi - lo > 1) {
-                const uint32_t mid = (lo + hi) / 2;
-                if (s_pref[mid] <= t) {
-                    lo = mid;
-                } else {
-                    hi = mid;
-                }
+        if (c1 < seglen) {
+            fetch(c1);
+            if (counter) {
+                count(c1, turn ^ 1U);
             }
-            fi                 = lo;
-            const int64_t u0   = s_ulo[fi] + static_cast<int64_t>(t - s_pref[fi]);
-            const int64_t uhi  = s_uhi[fi];
-            const RunGeom g    = s_geom[fi];
-            // bin of the unit: u0 mod nbins (a mask for power-of-two nbins, which holds
-            // for negative u0 too in two's complement)
-            const uint32_t b   = pow2 ? static_cast<uint32_t>(u0) & (nbins - 1U)
-                                      : static_cast<uint32_t>(((u0 % nb) + nb) % nb);
-            float2* slot       = acc + fi * nbins + b;
+        }
+        const uint32_t cols = ncol[turn];
+        const float inv     = 1.0F / static_cast<float>(cols);
+        for (uint32_t t = tid; t < nf * cols; t += kFoldBlock) {
+            // t / cols: below 2^16, where the rounded product is off by less than half
+            const uint32_t fi  = static_cast<uint32_t>((static_cast<float>(t) + 0.5F) * inv);
+            const uint32_t i   = t - fi * cols;
+            const UnitFreq& q  = fq[fi];
+            const UnitChunk& c = q.c[turn];
+            if (i >= c.cnt) {
+                continue;
+            }
+            const uint32_t b = c.b0 + i;
+            float2* slot     = acc + fi * nbins + (b >= nbins ? b - nbins : b);
             float ae = slot->x, av = slot->y;
-            for (int64_t u = u0; u <= uhi; u += nb) {
-                uint32_t a = run_bound(u, seglen, tsamp, t_ref, g, nbins);
-                uint32_t z = run_bound(u + 1, seglen, tsamp, t_ref, g, nbins);
-                a = a > c0 ? a : c0;
-                z = z < c1 ? z : c1;
-                uint32_t k = a;
-                if ((k & 1U) != 0 && k < z) {  // c0 is even: align to a sample pair
-                    const float2 x = s_ev[k - c0];
+            double u = static_cast<double>(i);
+            for (int64_t ui = c.ulo + i; ui <= c.uhi; ui += nb, u += static_cast<double>(nbins)) {
+                uint32_t k = unit_start<CHUNK>(q, c, u, c0, c1, seglen, tsamp, t_ref, nbins);
+                const uint32_t z =
+                    unit_start<CHUNK>(q, c, u + 1.0, c0, c1, seglen, tsamp, t_ref, nbins);
+                if ((k & 1U) != 0 && k < z) {  // align to a sample pair
+                    const float2 x = s_ev[k];
                     ae = ae + x.x;
                     av = av + x.y;
                     ++k;
@@ -288,36 +350,36 @@ __device__ __forceinline__ void bf_units_block(uint32_t bid, const float* __rest
                 // 16-byte reads of two (e, v) pairs (fewer LDS instructions, and 8 lanes
                 // per LDS pass instead of 16), 16 samples per step, then 8, then one by
                 // one: every sample is still added in ascending order
-                const auto* __restrict__ p = reinterpret_cast<const float4*>(s_ev) +
-                                              (k < z ? (k - c0) / 2 : 0);
                 const uint32_t npair = k < z ? (z - k) / 2 : 0;
+                const auto* __restrict__ p = reinterpret_cast<const float4*>(s_ev) +
+                                              (k < z ? k / 2 : 0);
                 const float4* const pend = p + npair;
                 for (; p + 8 <= pend; p += 8) {
                     float4 y[8];
 #pragma unroll
-                    for (int i = 0; i < 8; ++i) {
-                        y[i] = p[i];
+                    for (int w = 0; w < 8; ++w) {
+                        y[w] = p[w];
                     }
 #pragma unroll
-                    for (int i = 0; i < 8; ++i) {
-                        ae = ae + y[i].x;
-                        av = av + y[i].y;
-                        ae = ae + y[i].z;
-                        av = av + y[i].w;
+                    for (int w = 0; w < 8; ++w) {
+                        ae = ae + y[w].x;
+                        av = av + y[w].y;
+                        ae = ae + y[w].z;
+                        av = av + y[w].w;
                     }
                 }
                 if (p + 4 <= pend) {
                     float4 y[4];
 #pragma unroll
-                    for (int i = 0; i < 4; ++i) {
-                        y[i] = p[i];
+                    for (int w = 0; w < 4; ++w) {
+                        y[w] = p[w];
                     }
 #pragma unroll
-                    for (int i = 0; i < 4; ++i) {
-                        ae = ae + y[i].x;
-                        av = av + y[i].y;
-                        ae = ae + y[i].z;
-                        av = av + y[i].w;
+                    for (int w = 0; w < 4; ++w) {
+                        ae = ae + y[w].x;
+                        av = av + y[w].y;
+                        ae = ae + y[w].z;
+                        av = av + y[w].w;
                     }
                     p += 4;
                 }
@@ -330,7 +392,7 @@ __device__ __forceinline__ void bf_units_block(uint32_t bid, const float* __rest
                 }
                 k += 2 * npair;
                 if (k < z) {  // an odd last sample
-                    const float2 x = s_ev[k - c0];
+                    const float2 x = s_ev[k];
                     ae = ae + x.x;
                     av = av + x.y;
                 }

@@ -132,13 +132,13 @@ k_bf_fill(const double* __restrict__ freqs, uint32_t seglen, uint32_t nbins, dou
 }
 
 
-template <typename TO>
+template <typename TO, int CHUNK>
 __global__ void __launch_bounds__(kBlock)
 k_bf_units(const float* __restrict__ ts_e, const float* __restrict__ ts_v, uint32_t seglen,
            uint32_t nfreqs, uint32_t nbins, uint32_t blocks_per_seg,
            const double* __restrict__ freqs, double tsamp, double t_ref, TO* __restrict__ fold,
            float scale) {
-    bf_units_block<TO>(blockIdx.x, ts_e, ts_v, seglen, nfreqs, nbins, blocks_per_seg, freqs,
+    bf_units_block<TO, CHUNK>(blockIdx.x, ts_e, ts_v, seglen, nfreqs, nbins, blocks_per_seg, freqs,
                        tsamp, t_ref, fold, scale);
 }
 
@@ -357,6 +357,8 @@ unsigned char* scratch_address() {
 
 constexpr uint64_t align256(uint64_t x) { return (x + 255) & ~static_cast<uint64_t>(255); }
 
+constexpr uint64_t kUnitBlocks = 512;  // two per CU
+
 /// Segments per block of the list fold: as many as fit 32 KB of LDS (8 B per
 /// sample), at most 8; 1 selects the one-segment kernel.
 int fold_segs_per_block(uint32_t seglen) {
@@ -374,8 +376,15 @@ void launch_fold(const float* ts_e, const float* ts_v, uint64_t blocks, uint32_t
     if (L.use_runs) {
         const auto g = static_cast<unsigned>(blocks);
         const auto* fr = L.freqs;
-        k_bf_units<TO><<<g, kBlock, unit_lds_bytes(L.nbins), s>>>(
-            ts_e, ts_v, L.seglen, L.nfreqs, L.nbins, bps, fr, L.tsamp, L.t_ref, fold, scale);
+        if (blocks < 2 * kUnitBlocks) {
+            k_bf_units<TO, kUnitChunkSmall>
+                <<<g, kBlock, unit_lds_bytes(L.nbins, kUnitChunkSmall), s>>>(
+                    ts_e, ts_v, L.seglen, L.nfreqs, L.nbins, bps, fr, L.tsamp, L.t_ref, fold,
+                    scale);
+        } else {
+            k_bf_units<TO, kUnitChunk><<<g, kBlock, unit_lds_bytes(L.nbins), s>>>(
+                ts_e, ts_v, L.seglen, L.nfreqs, L.nbins, bps, fr, L.tsamp, L.t_ref, fold, scale);
+        }
     } else if (fold_segs_per_block(L.seglen) > 1) {
         // blocks = nseg * bps; the multi-segment grid covers ceil(nseg / NS) groups
         const uint64_t nseg = blocks / bps;
@@ -413,7 +422,7 @@ void brute_fold_time(const float* ts_e, const float* ts_v, uint64_t nseg,
 void brute_fold_time(const float* ts_e, const float* ts_v, uint64_t nseg,
                      const BruteFoldView& L, void* fold, FoldStorage so, float scale,
                      hipStream_t s) {
-    const uint32_t bps    = brute_fold_blocks_per_segment(L);
+    const uint32_t bps    = brute_fold_blocks_per_segment(L, nseg);
     const uint64_t blocks = nseg * bps;
     LOKI_REQUIRE(blocks < (1ULL << 31), "brute fold grid too large");
     if (blocks == 0) {
@@ -509,13 +518,19 @@ void brute_fold_time_noalloc(const float* ts_e, const float* ts_v, uint64_t nsam
     hip_check(hipStreamSynchronize(s), "brute fold");
 }
 
-uint32_t brute_fold_blocks_per_segment(const BruteFoldLists& L) {
-    return brute_fold_blocks_per_segment(L.view());
+uint32_t brute_fold_blocks_per_segment(const BruteFoldLists& L, uint64_t nseg) {
+    return brute_fold_blocks_per_segment(L.view(), nseg);
 }
 
-uint32_t brute_fold_blocks_per_segment(const BruteFoldView& L) {
+uint32_t brute_fold_blocks_per_segment(const BruteFoldView& L, uint64_t nseg) {
     if (L.use_runs) {
-        const uint32_t nf = unit_nf(L.nbins);
+        // Few segments: fewer frequencies per block, down to 8 (fewer leave too
+        // few units per chunk: 0.29 against 0.20 ms at 4 with 2^20 samples, 403
+        // frequencies, 64 bins), until there are two blocks per CU.
+        uint32_t nf = unit_nf(L.nbins);
+        while (nf > 8 && nseg * ((L.nfreqs + nf - 1) / nf) < kUnitBlocks) {
+            nf = (nf + 1) / 2;
+        }
         return (L.nfreqs + nf - 1) / nf;
     }
     const uint64_t pairs = static_cast<uint64_t>(L.nfreqs) * L.nbins;

@@ -329,8 +329,10 @@ void resolve_grouped(const ResolveTask* tasks, uint32_t ntasks, uint32_t nblocks
                      hipStream_t s);
 /// Blocks per segment of the time brute fold of `lists` (list or run path;
 /// tasks of one grouped launch must share the path).
-uint32_t brute_fold_blocks_per_segment(const BruteFoldLists& lists);
-uint32_t brute_fold_blocks_per_segment(const BruteFoldView& lists);
+/// nseg: segments the launch folds (all its tasks' together): few take more
+/// blocks each.
+uint32_t brute_fold_blocks_per_segment(const BruteFoldLists& lists, uint64_t nseg);
+uint32_t brute_fold_blocks_per_segment(const BruteFoldView& lists, uint64_t nseg);
 /// Grouped time brute fold (all tasks stored as `so`): the list path, or with
 /// `runs` the long-segment run path (max_nbins: the largest nbins of the
 /// tasks, which sizes its LDS).

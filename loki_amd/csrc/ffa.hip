@@ -370,20 +370,16 @@ void FFAExecutor::init_level(const float* ts_e, const float* ts_v, void* out, vo
 void* FFAExecutor::run_levels(const float* ts_e, const float* ts_v, void* buf_even,
                               void* buf_odd, SizeType last_level, bool last_fp32,
                               hipStream_t s, SizeType coords_level) {
-    // Level k lands in buf_even for even k and in buf_odd for odd k (the
-    // reference picks its ping-pong start side the same way so the last level
-    // lands in the caller's buffer, ffa.cpp:261-276).
+    // The last level lands in buf_even or buf_odd by its parity (the reference
+    // picks its ping-pong start side so that it is the caller's buffer,
+    // ffa.cpp:261-276); the side of level 0 follows from the number of passes.
     LOKI_REQUIRE(last_level < m_plan.n_levels(), "level out of range");
     m_timer.reset();
     m_ws->coords.reserve(m_plan.coord_size() * coord_record_bytes());
     prepare_brute_fold(s);
     resolve_coordinates(m_ws->coords.get(), s, std::max(last_level, coords_level));
 
-    void* even           = buf_even;
-    void* odd            = buf_odd;
     const SizeType nbins = m_plan.config().get_nbins();
-    init_level(ts_e, ts_v, even, odd, last_fp32 && last_level == 0, s);
-
     auto tables = [&](SizeType l, const FFACoord*& cp, const FFACoordFreq*& cfp) {
         const SizeType off = m_plan.ncoords_offsets64()[l];
         cp                 = nullptr;
@@ -395,12 +391,10 @@ void* FFAExecutor::run_levels(const float* ts_e, const float* ts_v, void* buf_ev
         }
     };
     // Pass plan: levels l and l + 1 merged in one two-level pass where allowed
-    // (time domain, both stored in the tree's storage), pairing from the top
-    // down; the number of two-level passes is kept even, so that level k
-    // still lands in buf_even for even k and in buf_odd for odd k.
+    // (Fourier, or both stored in the tree's storage), pairing from the top down.
     std::vector<uint8_t> two(last_level + 2, 0);  // two[l]: levels l, l+1 in one pass
-    if (!m_fourier && m_two_level && kern::merge2_supported(static_cast<uint32_t>(nbins))) {
-        std::vector<SizeType> starts;
+    SizeType passes = last_level;
+    if (m_two_level && (m_fourier || kern::merge2_supported(static_cast<uint32_t>(nbins)))) {
         for (SizeType top = last_level; top >= 2;) {
             const SizeType l     = top - 1;
             const FoldStorage si = stored_as(l - 1, last_level, last_fp32);
@@ -413,23 +407,25 @@ void* FFAExecutor::run_levels(const float* ts_e, const float* ts_v, void* buf_ev
             // than two single passes (2^23-sample accel search, levels 10-11:
             // 1.97 ms against 0.47 + 1.28 ms)
             const bool grows = m_plan.level_size(top) > m_plan.level_size(l - 1) + m_plan.level_size(l - 1) / 4;
-            if (to32 || grows || sb != so ||
-                !(si == so || (si == FoldStorage::kF32 && so == FoldStorage::kBFP16))) {
+            const bool storable =
+                m_fourier || (!to32 && sb == so &&
+                              (si == so || (si == FoldStorage::kF32 && so == FoldStorage::kBFP16)));
+            if (grows || !storable) {
                 top -= 1;  // this pair cannot be merged in one pass; try one lower
                 continue;
             }
-            starts.push_back(l);
+            two[l] = 1;
+            passes -= 1;
             top -= 2;
         }
-        if (starts.size() % 2 == 1) {
-            starts.pop_back();  // the lowest pair
-        }
-        for (const SizeType l : starts) {
-            two[l] = 1;
-        }
     }
-    void* cur   = even;
-    void* other = odd;
+    void* const last = last_level % 2 == 0 ? buf_even : buf_odd;
+    void* cur        = last;
+    void* other      = last_level % 2 == 0 ? buf_odd : buf_even;
+    if (passes % 2 == 1) {
+        std::swap(cur, other);
+    }
+    init_level(ts_e, ts_v, cur, other, last_fp32 && last_level == 0, s);
     for (SizeType l = 1; l <= last_level;) {
         const FFACoord* cp      = nullptr;
         const FFACoordFreq* cfp = nullptr;
@@ -439,11 +435,19 @@ void* FFAExecutor::run_levels(const float* ts_e, const float* ts_v, void* buf_ev
             const FFACoordFreq* cfp2 = nullptr;
             tables(l + 1, cp2, cfp2);
             const int slot = m_timer.start(KernelKind::kMerge, static_cast<int>(l + 1), s);
-            kern::merge_time2(cur, other, cp, cfp, cp2, cfp2, m_plan.ncoords()[l + 1],
-                              m_plan.ncoords()[l], m_plan.ncoords()[l - 1],
-                              m_plan.nsegments()[l + 1], m_plan.param_counts()[l + 1].back(),
-                              static_cast<uint32_t>(nbins), stored_as(l - 1, last_level, last_fp32),
-                              stored_as(l + 1, last_level, last_fp32), 0.5F, s);
+            if (m_fourier) {
+                kern::merge_fourier2(static_cast<const float2*>(cur), static_cast<float2*>(other),
+                                     cp, cfp, cp2, cfp2, m_plan.ncoords()[l + 1],
+                                     m_plan.ncoords()[l - 1], m_plan.nsegments()[l + 1],
+                                     static_cast<uint32_t>(nbins), s);
+            } else {
+                kern::merge_time2(cur, other, cp, cfp, cp2, cfp2, m_plan.ncoords()[l + 1],
+                                  m_plan.ncoords()[l], m_plan.ncoords()[l - 1],
+                                  m_plan.nsegments()[l + 1], m_plan.param_counts()[l + 1].back(),
+                                  static_cast<uint32_t>(nbins),
+                                  stored_as(l - 1, last_level, last_fp32),
+                                  stored_as(l + 1, last_level, last_fp32), 0.5F, s);
+            }
             check_launch("two-level merge launch");
             m_timer.stop(slot, s);
             l += 2;
@@ -473,7 +477,7 @@ void* FFAExecutor::run_levels(const float* ts_e, const float* ts_v, void* buf_ev
         }
         std::swap(cur, other);
     }
-    LOKI_REQUIRE(cur == ((last_level % 2 == 0) ? even : odd), "merge passes: wrong landing buffer");
+    LOKI_REQUIRE(cur == last, "merge passes: wrong landing buffer");
     return cur;
 }
 

@@ -19,9 +19,7 @@
 //   out[s, c, q, k] = in[2s, i_t, q, k] w(s_t)^k + in[2s+1, i_h, q, k] w(s_h)^k,
 //   w(x)^k = exp(-2 pi i k x / nbins) with the fractional shift x,
 // (freq-only: tail factor 1).  One lane per (segment, coordinate, harmonic)
-// handles both components; the angle k*x/nbins is reduced mod 1 in FP64 and
-// the twiddle comes from an accurate sincospi plus a first-order correction
-// for the FP32 rounding of the reduced angle.
+// handles both components of one level or of two in one pass.
 #include <hip/hip_runtime.h>
 
 #include <cmath>
@@ -539,60 +537,161 @@ __device__ __forceinline__ float2 cmul(float2 a, float2 w) {
     return make_float2(fmaf(a.x, w.x, -(a.y * w.y)), fmaf(a.x, w.y, a.y * w.x));
 }
 
-// IDX: uint32_t when nseg * ncur * nbf < 2^32 (cheaper index division), else uint64_t.
-template <bool POLY, typename IDX>
+/// exp(-2 pi i k s / nbins) of a shift s in [0, nbins) bins: the angle is
+/// reduced to an eighth of a turn about a quarter turn, then a polynomial each
+/// for sine and cosine (fitted to 3.4e-9 and 5e-11; 0.44 and 0.30 ulp rms with
+/// FP32 rounding).  POW2: k s as an exact FP32 pair, whose head scales and
+/// reduces exactly; otherwise in FP64.
+template <bool POW2>
+__device__ __forceinline__ float2 shift_twiddle(float s, float k, float inv_f, double inv_n) {
+    float q, f;
+    if constexpr (POW2) {
+        const float hi = k * s;
+        const float r  = hi * inv_f;
+        q              = rintf(4.0F * r);
+        f              = fmaf(fmaf(k, s, -hi), inv_f, fmaf(q, -0.25F, r));
+    } else {
+        const double d  = static_cast<double>(k) * static_cast<double>(s) * inv_n;
+        const double qd = rint(4.0 * d);
+        q               = static_cast<float>(qd);
+        f               = static_cast<float>(fma(qd, -0.25, d));
+    }
+    const float z  = f * f;
+    const float sp = fmaf(fmaf(fmaf(-7.540161270e+01F, z, 8.159254287e+01F), z, -4.134166257e+01F),
+                          z, -1.942122e-07F);
+    const float sn = fmaf(f, 6.2831855F, f * sp);
+    const float cs = fmaf(
+        fmaf(fmaf(fmaf(5.922016912e+01F, z, -8.544284468e+01F), z, 6.493931614e+01F), z,
+             -1.973920865e+01F),
+        z, 1.0F);
+    const auto iq    = static_cast<uint32_t>(static_cast<int32_t>(q));
+    const float x    = (iq & 1U) != 0 ? sn : cs;
+    const float y    = (iq & 1U) != 0 ? cs : sn;
+    const uint32_t m = 0x80000000U;
+    return make_float2(__uint_as_float(__float_as_uint(x) ^ (((iq + 1U) << 30) & m)),
+                       __uint_as_float(__float_as_uint(y) ^ ((~iq << 30) & m)));
+}
+
+/// Division of 32-bit numbers by a runtime constant d >= 1 (Granlund and
+/// Montgomery's multiplication by a precomputed reciprocal).
+struct FastDiv {
+    uint32_t d, mul, sh1, sh2;
+};
+FastDiv fast_div(uint64_t d) {
+    uint32_t l = 0;
+    while ((1ULL << l) < d) {
+        ++l;
+    }
+    FastDiv f;
+    f.d   = static_cast<uint32_t>(d);
+    f.mul = static_cast<uint32_t>(((1ULL << 32) * ((1ULL << l) - d)) / d + 1);
+    f.sh1 = l < 1 ? l : 1;
+    f.sh2 = l < 1 ? 0 : l - 1;
+    return f;
+}
+__device__ __forceinline__ uint32_t div_by(uint32_t n, const FastDiv& f) {
+    const uint32_t t = __umulhi(n, f.mul);
+    return (t + ((n - t) >> f.sh1)) >> f.sh2;
+}
+
+struct FourierMergeArgs {
+    const float2* in;
+    float2* out;
+    const FFACoord* coords;         // poly levels
+    const FFACoordFreq* cf;         // freq-only levels
+    const FFACoord* coords_up;      // two levels: the upper level's records
+    const FFACoordFreq* cf_up;
+    uint64_t ncur, nprev, nseg;     // output level; input level's coordinates
+    uint32_t nbf;
+    FastDiv by_nbf, by_ncur;
+    float inv_f;
+    double inv_n;
+};
+
+struct FourierPair {
+    float2 e, v;
+};
+
+__device__ __forceinline__ FourierPair load_pair(const float2* in, uint64_t row, uint32_t nbf,
+                                                 uint32_t k) {
+    const float2* r = in + row * 2 * nbf + k;
+    return {r[0], r[nbf]};
+}
+
+/// tail w(st) + head w(sh) of both components (freq-only: the tail unturned).
+template <bool POLY, bool POW2>
+__device__ __forceinline__ FourierPair merge_pair(const FourierMergeArgs& a, const FourierPair& t,
+                                                  const FourierPair& h, float st, float sh,
+                                                  float k) {
+    const float2 wh = shift_twiddle<POW2>(sh, k, a.inv_f, a.inv_n);
+    const float2 he = cmul(h.e, wh);
+    const float2 hv = cmul(h.v, wh);
+    float2 te = t.e, tv = t.v;
+    if constexpr (POLY) {
+        const float2 wt = shift_twiddle<POW2>(st, k, a.inv_f, a.inv_n);
+        te              = cmul(te, wt);
+        tv              = cmul(tv, wt);
+    }
+    return {make_float2(te.x + he.x, te.y + he.y), make_float2(tv.x + hv.x, tv.y + hv.y)};
+}
+
+template <bool POLY>
+__device__ __forceinline__ FFACoord record_of(const FFACoord* coords, const FFACoordFreq* cf,
+                                              uint64_t c) {
+    if constexpr (POLY) {
+        return coords[c];
+    } else {
+        const FFACoordFreq r = cf[c];
+        return {r.idx, 0.0F, r.idx, r.shift};
+    }
+}
+
+// IDX: uint32_t when nseg * ncur * nbf < 2^32 (division by multiplication),
+// else uint64_t.  LEVELS 2: the output level's parents are formed from their
+// own parents (four rows) in registers and never stored.  2^22 samples, 33
+// harmonics (2.0 GB per level): 0.87 ms for one level, 1.0 ms for two in one
+// pass against 0.90 ms each; HBM-bound, and before the short twiddles about
+// half the time went into FP64 angles and sincospi.
+template <int LEVELS, bool POLY, bool POW2, typename IDX>
 __global__ void __launch_bounds__(kBlock)
-k_merge_fourier(const float2* __restrict__ in, float2* __restrict__ out,
-                const FFACoord* __restrict__ coords, const FFACoordFreq* __restrict__ cf,
-                IDX ncur, uint64_t nprev, IDX nseg, uint32_t nbf, uint32_t nbins) {
-    const IDX total    = nseg * ncur * nbf;
-    const double inv_n = 1.0 / static_cast<double>(nbins);
+k_merge_fourier(FourierMergeArgs a) {
+    const IDX ncur  = static_cast<IDX>(a.ncur);
+    const IDX total = static_cast<IDX>(a.nseg) * ncur * a.nbf;
     for (IDX t = static_cast<IDX>(blockIdx.x) * kBlock + threadIdx.x; t < total;
          t += static_cast<IDX>(gridDim.x) * kBlock) {
-        const uint32_t k   = static_cast<uint32_t>(t % nbf);
-        const IDX r        = t / nbf;
-        const uint64_t c   = r % ncur;
-        const uint64_t seg = r / ncur;
-        uint64_t it_row, ih_row;
-        float st = 0.0F, sh;
-        if constexpr (POLY) {
-            const FFACoord cd = coords[c];
-            it_row = (2 * seg) * nprev + cd.i_tail;
-            ih_row = (2 * seg + 1) * nprev + cd.i_head;
-            st     = cd.shift_tail;
-            sh     = cd.shift_head;
+        IDX r, seg;
+        if constexpr (sizeof(IDX) == 4) {
+            r   = div_by(t, a.by_nbf);
+            seg = div_by(r, a.by_ncur);
         } else {
-            const FFACoordFreq cd = cf[c];
-            it_row = (2 * seg) * nprev + cd.idx;
-            ih_row = (2 * seg + 1) * nprev + cd.idx;
-            sh     = cd.shift;
+            r   = t / a.nbf;
+            seg = r / ncur;
         }
-        const float2* tr = in + it_row * 2 * nbf;
-        const float2* hr = in + ih_row * 2 * nbf;
-        const float2 te  = tr[k];
-        const float2 tv  = tr[nbf + k];
-        const float2 he  = hr[k];
-        const float2 hv  = hr[nbf + k];
-        const double kd  = static_cast<double>(k);
-        const float2 wh  = twiddle_turns(kd * static_cast<double>(sh) * inv_n);
-        float2 oe, ov;
-        if constexpr (POLY) {
-            const float2 wt = twiddle_turns(kd * static_cast<double>(st) * inv_n);
-            const float2 a  = cmul(te, wt);
-            const float2 b  = cmul(he, wh);
-            const float2 cc = cmul(tv, wt);
-            const float2 d  = cmul(hv, wh);
-            oe = make_float2(a.x + b.x, a.y + b.y);
-            ov = make_float2(cc.x + d.x, cc.y + d.y);
+        const uint32_t k  = static_cast<uint32_t>(t - r * a.nbf);
+        const uint64_t c  = r - seg * ncur;
+        const auto kf     = static_cast<float>(k);
+        FourierPair o;
+        if constexpr (LEVELS == 1) {
+            const FFACoord cd   = record_of<POLY>(a.coords, a.cf, c);
+            const FourierPair p = load_pair(a.in, (2 * seg) * a.nprev + cd.i_tail, a.nbf, k);
+            const FourierPair q = load_pair(a.in, (2 * seg + 1) * a.nprev + cd.i_head, a.nbf, k);
+            o = merge_pair<POLY, POW2>(a, p, q, cd.shift_tail, cd.shift_head, kf);
         } else {
-            const float2 b = cmul(he, wh);
-            const float2 d = cmul(hv, wh);
-            oe = make_float2(te.x + b.x, te.y + b.y);
-            ov = make_float2(tv.x + d.x, tv.y + d.y);
+            const FFACoord up = record_of<POLY>(a.coords_up, a.cf_up, c);
+            const FFACoord lt = record_of<POLY>(a.coords, a.cf, up.i_tail);
+            const FFACoord lh = record_of<POLY>(a.coords, a.cf, up.i_head);
+            const uint64_t s4 = static_cast<uint64_t>(seg) * 4 * a.nprev;
+            const FourierPair p0 = load_pair(a.in, s4 + lt.i_tail, a.nbf, k);
+            const FourierPair p1 = load_pair(a.in, s4 + a.nprev + lt.i_head, a.nbf, k);
+            const FourierPair p2 = load_pair(a.in, s4 + 2 * a.nprev + lh.i_tail, a.nbf, k);
+            const FourierPair p3 = load_pair(a.in, s4 + 3 * a.nprev + lh.i_head, a.nbf, k);
+            const FourierPair mt = merge_pair<POLY, POW2>(a, p0, p1, lt.shift_tail, lt.shift_head, kf);
+            const FourierPair mh = merge_pair<POLY, POW2>(a, p2, p3, lh.shift_tail, lh.shift_head, kf);
+            o = merge_pair<POLY, POW2>(a, mt, mh, up.shift_tail, up.shift_head, kf);
         }
-        float2* o = out + (seg * ncur + c) * 2 * nbf;
-        o[k]       = oe;
-        o[nbf + k] = ov;
+        float2* w = a.out + (static_cast<uint64_t>(seg) * a.ncur + c) * 2 * a.nbf + k;
+        w[0]      = o.e;
+        w[a.nbf]  = o.v;
     }
 }
 
@@ -717,38 +816,87 @@ void brute_fold_fourier(const float* ts_e, const float* ts_v, uint64_t nseg, uin
     }
 }
 
+namespace {
+
+template <int LEVELS, bool POLY>
+void launch_merge_fourier(const FourierMergeArgs& a, bool pow2, uint64_t total, hipStream_t s) {
+    const unsigned g = grid_for(total);
+    // the grid-stride loop must not overflow the index type
+    const bool narrow = total + static_cast<uint64_t>(g) * kBlock < (1ULL << 32);
+    if (pow2) {
+        if (narrow) {
+            k_merge_fourier<LEVELS, POLY, true, uint32_t><<<g, kBlock, 0, s>>>(a);
+        } else {
+            k_merge_fourier<LEVELS, POLY, true, uint64_t><<<g, kBlock, 0, s>>>(a);
+        }
+    } else if (narrow) {
+        k_merge_fourier<LEVELS, POLY, false, uint32_t><<<g, kBlock, 0, s>>>(a);
+    } else {
+        k_merge_fourier<LEVELS, POLY, false, uint64_t><<<g, kBlock, 0, s>>>(a);
+    }
+}
+
+FourierMergeArgs fourier_merge_args(const float2* in, float2* out, uint64_t ncur, uint64_t nprev,
+                                    uint64_t nseg, uint32_t nbins) {
+    LOKI_REQUIRE(nbins >= 1, "merge: nbins must be positive");
+    FourierMergeArgs a{};
+    a.in      = in;
+    a.out     = out;
+    a.ncur    = ncur;
+    a.nprev   = nprev;
+    a.nseg    = nseg;
+    a.nbf     = nbins / 2 + 1;
+    a.by_nbf  = fast_div(a.nbf);
+    a.by_ncur = fast_div(ncur < (1ULL << 32) ? ncur : 1);  // unused beyond 32 bits
+    a.inv_n   = 1.0 / static_cast<double>(nbins);
+    a.inv_f   = static_cast<float>(a.inv_n);
+    return a;
+}
+
+}  // namespace
+
 void merge_fourier(const float2* in, float2* out, const FFACoord* coords,
                    const FFACoordFreq* coords_freq, uint64_t ncur, uint64_t nprev, uint64_t nseg,
                    uint32_t nbins, hipStream_t s) {
-    LOKI_REQUIRE(nbins >= 1, "merge: nbins must be positive");
     LOKI_REQUIRE((coords == nullptr) != (coords_freq == nullptr),
                  "merge: exactly one coordinate table");
     if (ncur == 0 || nseg == 0) {
         return;
     }
-    const uint32_t nbf   = nbins / 2 + 1;
-    const uint64_t total = nseg * ncur * nbf;
-    const unsigned g     = grid_for(total);
-    // the grid-stride loop must not overflow the index type
-    const bool narrow = total + static_cast<uint64_t>(g) * kBlock < (1ULL << 32);
+    auto a              = fourier_merge_args(in, out, ncur, nprev, nseg, nbins);
+    a.coords            = coords;
+    a.cf                = coords_freq;
+    const bool pow2     = (nbins & (nbins - 1)) == 0;
+    const uint64_t size = nseg * ncur * a.nbf;
     if (coords != nullptr) {
-        if (narrow) {
-            k_merge_fourier<true, uint32_t><<<g, kBlock, 0, s>>>(
-                in, out, coords, nullptr, static_cast<uint32_t>(ncur), nprev,
-                static_cast<uint32_t>(nseg), nbf, nbins);
-        } else {
-            k_merge_fourier<true, uint64_t><<<g, kBlock, 0, s>>>(in, out, coords, nullptr, ncur,
-                                                                 nprev, nseg, nbf, nbins);
-        }
+        launch_merge_fourier<1, true>(a, pow2, size, s);
     } else {
-        if (narrow) {
-            k_merge_fourier<false, uint32_t><<<g, kBlock, 0, s>>>(
-                in, out, nullptr, coords_freq, static_cast<uint32_t>(ncur), nprev,
-                static_cast<uint32_t>(nseg), nbf, nbins);
-        } else {
-            k_merge_fourier<false, uint64_t><<<g, kBlock, 0, s>>>(
-                in, out, nullptr, coords_freq, ncur, nprev, nseg, nbf, nbins);
-        }
+        launch_merge_fourier<1, false>(a, pow2, size, s);
+    }
+}
+
+void merge_fourier2(const float2* in, float2* out, const FFACoord* coords,
+                    const FFACoordFreq* coords_freq, const FFACoord* coords_up,
+                    const FFACoordFreq* coords_freq_up, uint64_t ncur, uint64_t nprev,
+                    uint64_t nseg, uint32_t nbins, hipStream_t s) {
+    LOKI_REQUIRE((coords == nullptr) != (coords_freq == nullptr) &&
+                     (coords == nullptr) == (coords_up == nullptr) &&
+                     (coords_freq == nullptr) == (coords_freq_up == nullptr),
+                 "merge: exactly one coordinate table per level");
+    if (ncur == 0 || nseg == 0) {
+        return;
+    }
+    auto a              = fourier_merge_args(in, out, ncur, nprev, nseg, nbins);
+    a.coords            = coords;
+    a.cf                = coords_freq;
+    a.coords_up         = coords_up;
+    a.cf_up             = coords_freq_up;
+    const bool pow2     = (nbins & (nbins - 1)) == 0;
+    const uint64_t size = nseg * ncur * a.nbf;
+    if (coords != nullptr) {
+        launch_merge_fourier<2, true>(a, pow2, size, s);
+    } else {
+        launch_merge_fourier<2, false>(a, pow2, size, s);
     }
 }
 

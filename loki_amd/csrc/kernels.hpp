@@ -158,6 +158,14 @@ void merge_fourier(const float2* in, float2* out, const FFACoord* coords,
                    const FFACoordFreq* coords_freq, uint64_t ncur, uint64_t nprev, uint64_t nseg,
                    uint32_t nbins, hipStream_t s);
 
+/// Two levels in one pass, the same values as two merge_fourier calls: coords
+/// of the lower level, coords_up of the upper (output) level, ncur its
+/// coordinates and nseg its segments, nprev the input level's coordinates.
+void merge_fourier2(const float2* in, float2* out, const FFACoord* coords,
+                    const FFACoordFreq* coords_freq, const FFACoord* coords_up,
+                    const FFACoordFreq* coords_freq_up, uint64_t ncur, uint64_t nprev,
+                    uint64_t nseg, uint32_t nbins, hipStream_t s);
+
 /// Inverse real DFT of nrows rows of nbins/2+1 float2 into rows of nbins
 /// floats, scaled by 1/nbins (C2R + normalisation).
 void irfft_rows(const float2* in, float* out, uint64_t nrows, uint32_t nbins, hipStream_t s);

@@ -612,25 +612,33 @@ struct FourierPair {
     float2 e, v;
 };
 
-__device__ __forceinline__ FourierPair load_pair(const float2* in, uint64_t row, uint32_t nbf,
-                                                 uint32_t k) {
-    const float2* r = in + row * 2 * nbf + k;
+__device__ __forceinline__ FourierPair load_pair(const float2* r, uint32_t nbf) {
     return {r[0], r[nbf]};
 }
 
-/// tail w(st) + head w(sh) of both components (freq-only: the tail unturned).
+/// Twiddles of one coordinate's tail and head (freq-only: the tail unturned).
+struct TwiddlePair {
+    float2 t, h;
+};
 template <bool POLY, bool POW2>
-__device__ __forceinline__ FourierPair merge_pair(const FourierMergeArgs& a, const FourierPair& t,
-                                                  const FourierPair& h, float st, float sh,
-                                                  float k) {
-    const float2 wh = shift_twiddle<POW2>(sh, k, a.inv_f, a.inv_n);
-    const float2 he = cmul(h.e, wh);
-    const float2 hv = cmul(h.v, wh);
+__device__ __forceinline__ TwiddlePair twiddle_pair(const FourierMergeArgs& a, const FFACoord& c,
+                                                    float k) {
+    TwiddlePair w;
+    w.h = shift_twiddle<POW2>(c.shift_head, k, a.inv_f, a.inv_n);
+    w.t = POLY ? shift_twiddle<POW2>(c.shift_tail, k, a.inv_f, a.inv_n) : make_float2(1.0F, 0.0F);
+    return w;
+}
+
+/// Turned tail + turned head of both components.
+template <bool POLY>
+__device__ __forceinline__ FourierPair merge_pair(const FourierPair& t, const FourierPair& h,
+                                                  const TwiddlePair& w) {
+    const float2 he = cmul(h.e, w.h);
+    const float2 hv = cmul(h.v, w.h);
     float2 te = t.e, tv = t.v;
     if constexpr (POLY) {
-        const float2 wt = shift_twiddle<POW2>(st, k, a.inv_f, a.inv_n);
-        te              = cmul(te, wt);
-        tv              = cmul(tv, wt);
+        te = cmul(te, w.t);
+        tv = cmul(tv, w.t);
     }
     return {make_float2(te.x + he.x, te.y + he.y), make_float2(tv.x + hv.x, tv.y + hv.y)};
 }
@@ -648,50 +656,73 @@ __device__ __forceinline__ FFACoord record_of(const FFACoord* coords, const FFAC
 
 // IDX: uint32_t when nseg * ncur * nbf < 2^32 (division by multiplication),
 // else uint64_t.  LEVELS 2: the output level's parents are formed from their
-// own parents (four rows) in registers and never stored.  2^22 samples, 33
-// harmonics (2.0 GB per level): 0.87 ms for one level, 1.0 ms for two in one
-// pass against 0.90 ms each; HBM-bound, and before the short twiddles about
-// half the time went into FP64 angles and sincospi.
-template <int LEVELS, bool POLY, bool POW2, typename IDX>
+// own parents (four rows) in registers and never stored.  SEGS: segments per
+// lane; their records, twiddles and row offsets are the same.  Consecutive
+// rows share parents and stay in one XCD's L2 (xcd_remap).  2^22 samples, 33
+// harmonics, 2.0 GB per level: one level 0.85 ms (0.90 before), two levels in
+// one pass 1.12 ms with four segments per lane, 1.31 ms with one, whose
+// VALU work (six twiddles per value, 1.0 ms) is then the bound.
+template <int LEVELS, int SEGS, bool POLY, bool POW2, typename IDX>
 __global__ void __launch_bounds__(kBlock)
 k_merge_fourier(FourierMergeArgs a) {
     const IDX ncur  = static_cast<IDX>(a.ncur);
-    const IDX total = static_cast<IDX>(a.nseg) * ncur * a.nbf;
-    for (IDX t = static_cast<IDX>(blockIdx.x) * kBlock + threadIdx.x; t < total;
-         t += static_cast<IDX>(gridDim.x) * kBlock) {
-        IDX r, seg;
+    const IDX total = static_cast<IDX>(a.nseg / SEGS) * ncur * a.nbf;
+    for (IDX t = static_cast<IDX>(xcd_remap(blockIdx.x, gridDim.x)) * kBlock + threadIdx.x;
+         t < total; t += static_cast<IDX>(gridDim.x) * kBlock) {
+        IDX r, sg;
         if constexpr (sizeof(IDX) == 4) {
-            r   = div_by(t, a.by_nbf);
-            seg = div_by(r, a.by_ncur);
+            r  = div_by(t, a.by_nbf);
+            sg = div_by(r, a.by_ncur);
         } else {
-            r   = t / a.nbf;
-            seg = r / ncur;
+            r  = t / a.nbf;
+            sg = r / ncur;
         }
-        const uint32_t k  = static_cast<uint32_t>(t - r * a.nbf);
-        const uint64_t c  = r - seg * ncur;
-        const auto kf     = static_cast<float>(k);
-        FourierPair o;
+        const uint32_t k   = static_cast<uint32_t>(t - r * a.nbf);
+        const uint64_t c   = r - sg * ncur;
+        const uint64_t seg = static_cast<uint64_t>(sg) * SEGS;
+        const auto kf      = static_cast<float>(k);
+        const uint64_t row = 2ULL * a.nbf;  // complex values per row
+        float2* w          = a.out + (seg * a.ncur + c) * row + k;
         if constexpr (LEVELS == 1) {
-            const FFACoord cd   = record_of<POLY>(a.coords, a.cf, c);
-            const FourierPair p = load_pair(a.in, (2 * seg) * a.nprev + cd.i_tail, a.nbf, k);
-            const FourierPair q = load_pair(a.in, (2 * seg + 1) * a.nprev + cd.i_head, a.nbf, k);
-            o = merge_pair<POLY, POW2>(a, p, q, cd.shift_tail, cd.shift_head, kf);
+            const FFACoord cd    = record_of<POLY>(a.coords, a.cf, c);
+            const TwiddlePair tw = twiddle_pair<POLY, POW2>(a, cd, kf);
+            const float2* pt     = a.in + ((2 * seg) * a.nprev + cd.i_tail) * row + k;
+            const float2* ph     = a.in + ((2 * seg + 1) * a.nprev + cd.i_head) * row + k;
+#pragma unroll
+            for (int i = 0; i < SEGS; ++i) {
+                const FourierPair o =
+                    merge_pair<POLY>(load_pair(pt, a.nbf), load_pair(ph, a.nbf), tw);
+                w[0]     = o.e;
+                w[a.nbf] = o.v;
+                pt += 2 * a.nprev * row;
+                ph += 2 * a.nprev * row;
+                w += a.ncur * row;
+            }
         } else {
-            const FFACoord up = record_of<POLY>(a.coords_up, a.cf_up, c);
-            const FFACoord lt = record_of<POLY>(a.coords, a.cf, up.i_tail);
-            const FFACoord lh = record_of<POLY>(a.coords, a.cf, up.i_head);
-            const uint64_t s4 = static_cast<uint64_t>(seg) * 4 * a.nprev;
-            const FourierPair p0 = load_pair(a.in, s4 + lt.i_tail, a.nbf, k);
-            const FourierPair p1 = load_pair(a.in, s4 + a.nprev + lt.i_head, a.nbf, k);
-            const FourierPair p2 = load_pair(a.in, s4 + 2 * a.nprev + lh.i_tail, a.nbf, k);
-            const FourierPair p3 = load_pair(a.in, s4 + 3 * a.nprev + lh.i_head, a.nbf, k);
-            const FourierPair mt = merge_pair<POLY, POW2>(a, p0, p1, lt.shift_tail, lt.shift_head, kf);
-            const FourierPair mh = merge_pair<POLY, POW2>(a, p2, p3, lh.shift_tail, lh.shift_head, kf);
-            o = merge_pair<POLY, POW2>(a, mt, mh, up.shift_tail, up.shift_head, kf);
+            const FFACoord up    = record_of<POLY>(a.coords_up, a.cf_up, c);
+            const FFACoord lt    = record_of<POLY>(a.coords, a.cf, up.i_tail);
+            const FFACoord lh    = record_of<POLY>(a.coords, a.cf, up.i_head);
+            const TwiddlePair tt = twiddle_pair<POLY, POW2>(a, lt, kf);
+            const TwiddlePair th = twiddle_pair<POLY, POW2>(a, lh, kf);
+            const TwiddlePair tu = twiddle_pair<POLY, POW2>(a, up, kf);
+            const float2* base   = a.in + seg * 4 * a.nprev * row + k;
+            const float2* p0     = base + lt.i_tail * row;
+            const float2* p1     = base + (a.nprev + lt.i_head) * row;
+            const float2* p2     = base + (2 * a.nprev + lh.i_tail) * row;
+            const float2* p3     = base + (3 * a.nprev + lh.i_head) * row;
+#pragma unroll
+            for (int i = 0; i < SEGS; ++i) {
+                const uint64_t off   = static_cast<uint64_t>(i) * 4 * a.nprev * row;
+                const FourierPair mt = merge_pair<POLY>(load_pair(p0 + off, a.nbf),
+                                                        load_pair(p1 + off, a.nbf), tt);
+                const FourierPair mh = merge_pair<POLY>(load_pair(p2 + off, a.nbf),
+                                                        load_pair(p3 + off, a.nbf), th);
+                const FourierPair o  = merge_pair<POLY>(mt, mh, tu);
+                w[0]                 = o.e;
+                w[a.nbf]             = o.v;
+                w += a.ncur * row;
+            }
         }
-        float2* w = a.out + (static_cast<uint64_t>(seg) * a.ncur + c) * 2 * a.nbf + k;
-        w[0]      = o.e;
-        w[a.nbf]  = o.v;
     }
 }
 
@@ -818,21 +849,33 @@ void brute_fold_fourier(const float* ts_e, const float* ts_v, uint64_t nseg, uin
 
 namespace {
 
-template <int LEVELS, bool POLY>
-void launch_merge_fourier(const FourierMergeArgs& a, bool pow2, uint64_t total, hipStream_t s) {
-    const unsigned g = grid_for(total);
-    // the grid-stride loop must not overflow the index type
-    const bool narrow = total + static_cast<uint64_t>(g) * kBlock < (1ULL << 32);
+template <int LEVELS, int SEGS, bool POLY, typename IDX>
+void launch_merge_fourier_segs(const FourierMergeArgs& a, bool pow2, unsigned g, hipStream_t s) {
     if (pow2) {
-        if (narrow) {
-            k_merge_fourier<LEVELS, POLY, true, uint32_t><<<g, kBlock, 0, s>>>(a);
-        } else {
-            k_merge_fourier<LEVELS, POLY, true, uint64_t><<<g, kBlock, 0, s>>>(a);
-        }
-    } else if (narrow) {
-        k_merge_fourier<LEVELS, POLY, false, uint32_t><<<g, kBlock, 0, s>>>(a);
+        k_merge_fourier<LEVELS, SEGS, POLY, true, IDX><<<g, kBlock, 0, s>>>(a);
     } else {
-        k_merge_fourier<LEVELS, POLY, false, uint64_t><<<g, kBlock, 0, s>>>(a);
+        k_merge_fourier<LEVELS, SEGS, POLY, false, IDX><<<g, kBlock, 0, s>>>(a);
+    }
+}
+
+template <int LEVELS, bool POLY>
+void launch_merge_fourier(const FourierMergeArgs& a, bool pow2, hipStream_t s) {
+    const uint64_t total = a.nseg * a.ncur * a.nbf;
+    // the grid-stride loop must not overflow the index type
+    const bool narrow =
+        total + static_cast<uint64_t>(grid_for(total)) * kBlock < (1ULL << 32) &&
+        a.ncur < (1ULL << 32);
+    // Segments per lane: 4 while that leaves 16 waves per SIMD's worth of lanes
+    // (2^20), 2 while it leaves as many.
+    constexpr uint64_t kLanes = 1ULL << 20;
+    if (!narrow) {
+        launch_merge_fourier_segs<LEVELS, 1, POLY, uint64_t>(a, pow2, grid_for(total), s);
+    } else if (a.nseg % 4 == 0 && total / 4 >= kLanes) {
+        launch_merge_fourier_segs<LEVELS, 4, POLY, uint32_t>(a, pow2, grid_for(total / 4), s);
+    } else if (a.nseg % 2 == 0 && total / 2 >= kLanes) {
+        launch_merge_fourier_segs<LEVELS, 2, POLY, uint32_t>(a, pow2, grid_for(total / 2), s);
+    } else {
+        launch_merge_fourier_segs<LEVELS, 1, POLY, uint32_t>(a, pow2, grid_for(total), s);
     }
 }
 
@@ -867,11 +910,10 @@ void merge_fourier(const float2* in, float2* out, const FFACoord* coords,
     a.coords            = coords;
     a.cf                = coords_freq;
     const bool pow2     = (nbins & (nbins - 1)) == 0;
-    const uint64_t size = nseg * ncur * a.nbf;
     if (coords != nullptr) {
-        launch_merge_fourier<1, true>(a, pow2, size, s);
+        launch_merge_fourier<1, true>(a, pow2, s);
     } else {
-        launch_merge_fourier<1, false>(a, pow2, size, s);
+        launch_merge_fourier<1, false>(a, pow2, s);
     }
 }
 
@@ -892,11 +934,10 @@ void merge_fourier2(const float2* in, float2* out, const FFACoord* coords,
     a.coords_up         = coords_up;
     a.cf_up             = coords_freq_up;
     const bool pow2     = (nbins & (nbins - 1)) == 0;
-    const uint64_t size = nseg * ncur * a.nbf;
     if (coords != nullptr) {
-        launch_merge_fourier<2, true>(a, pow2, size, s);
+        launch_merge_fourier<2, true>(a, pow2, s);
     } else {
-        launch_merge_fourier<2, false>(a, pow2, size, s);
+        launch_merge_fourier<2, false>(a, pow2, s);
     }
 }
 

@@ -3,16 +3,29 @@
 // final fold row runs on the matrix cores as [rows x (re, im of nbins/2+1
 // harmonics)] x [(re, im) x nbins] (v_mfma_f32_16x16x4f32), the profile
 // p = e / sqrt(v) is formed from the accumulators, and the S/N of
-// score.cpp:95-172 is taken from a per-lane LDS prefix-sum row.  The time-domain final
-// fold (2 * nbins floats per trial) is never written.
+// score.cpp:95-172 is taken from a per-lane prefix sum.  The time-domain final fold
+// (2 * nbins floats per trial) is never written.
 //
 // One wave owns 64 consecutive trials: 8 MFMA tiles of 8 trials (16 rows:
-// trial-major, e before v) whose Fourier rows are staged contiguously in LDS,
-// then one lane per trial for the prefix sum and width maxima.
+// trial-major, e before v), then one lane per trial for the prefix sum and the
+// width maxima.  Neither memory (0.40 ms at the copy rate for 3.87e6 trials of 64
+// bins and 10 widths) nor the matrix cores (0.43 ms) nor the vector unit (0.28 ms)
+// bounds it alone; the waits between them do, so:
+//  - the A operands come straight from the rows into registers, one tile ahead,
+//    with the harmonics ordered for float2 loads (the basis is permuted alike);
+//    staged through LDS instead: 1.40 ms;
+//  - the basis stays in registers (read from the LDS table for each tile before);
+//  - the prefix sum stays in registers and every width has its own code with
+//    compile-time offsets, 1.5 operations per bin; widths from the LDS row with the
+//    rest alike: 1.38 ms.
+// 0.92 ms at that size; 1.83 ms with staged tiles, basis and widths from LDS and the
+// general division sequences.  Two waves per SIMD: a third needs 168 registers,
+// which spill (0.12 ms slower).
 #include <hip/hip_runtime.h>
 
 #include <cfloat>
 #include <cmath>
+#include <utility>
 
 #include "kernels.hpp"
 #include "score_device.hpp"
@@ -32,11 +45,11 @@ __device__ __forceinline__ void wave_sync() {
 }
 
 template <int NB> struct IrsGeom {
-    static constexpr int kNh   = NB / 2 + 1;
-    static constexpr int kRow  = 2 * kNh;                 // floats per component row
-    static constexpr int kKs   = (kRow + 3) / 4;          // K steps of 4
-    static constexpr int kNt   = NB / 16;                 // N tiles of 16 bins
-    static constexpr int kTile = kTileTrials * 2 * kRow;  // floats per staged tile
+    static constexpr int kNh  = NB / 2 + 1;
+    static constexpr int kRow = 2 * kNh;     // floats per component row
+    static constexpr int kF2  = NB / 8;      // float2 loads per lane and tile
+    static constexpr int kKs  = 2 * kF2 + 1; // K steps of 4
+    static constexpr int kNt  = NB / 16;     // N tiles of 16 bins
 };
 
 /// Inverse real DFT basis entry B[k][n] (k = 2h + {0: re, 1: im}):
@@ -44,7 +57,7 @@ template <int NB> struct IrsGeom {
 /// and h = NB/2 (whose imaginary parts are ignored), 2/NB otherwise, 0 for
 /// the padding k >= nbins + 2.  tw[t] = (cos, sin)(2 pi t / NB).
 template <int NB>
-__device__ __forceinline__ float irdft_basis(const float2* tw, int k, int n, int zero) {
+__device__ __forceinline__ float irdft_basis(const float2* tw, int k, int n) {
     constexpr int kRow = IrsGeom<NB>::kRow;
     const int h        = k >> 1;
     const bool edge    = h == 0 || h == NB / 2;
@@ -52,19 +65,45 @@ __device__ __forceinline__ float irdft_basis(const float2* tw, int k, int n, int
     const float c      = (k >= kRow || (imag && edge)) ? 0.0F
                          : edge                        ? 1.0F / static_cast<float>(NB)
                                                        : 2.0F / static_cast<float>(NB);
-    const float2 w     = tw[((h * n) & (NB - 1)) + zero];
+    const float2 w     = tw[(h * n) & (NB - 1)];
     return c * (imag ? -w.y : w.x);
 }
 
+/// max_j (psum[j + W] - psum[j]) of the circular prefix sum, psum[i] for i >=
+/// NB being psum[i - NB] + psum[NB - 1].
+template <int NB, int W>
+__device__ __forceinline__ float window_max_fixed(const float (&ps)[NB]) {
+    float ma = -FLT_MAX, mb = -FLT_MAX;
+#pragma unroll
+    for (int j = 0; j < NB; ++j) {
+        const float hi = (j + W < NB) ? ps[(j + W) % NB] : ps[(j + W - NB) % NB] + ps[NB - 1];
+        if ((j & 2) == 0) {
+            ma = __builtin_fmaxf(ma, hi - ps[j]);
+        } else {
+            mb = __builtin_fmaxf(mb, hi - ps[j]);
+        }
+    }
+    return __builtin_fmaxf(ma, mb);
+}
+
+template <int NB, int... Ws>
+__device__ __forceinline__ float window_max_reg(std::integer_sequence<int, Ws...>,
+                                                const float (&ps)[NB], uint32_t w) {
+    float r = 0.0F;
+    (void)((w == static_cast<uint32_t>(Ws + 1) ? (r = window_max_fixed<NB, Ws + 1>(ps), true)
+                                               : false) ||
+           ...);
+    return r;
+}
+
 template <int NB, bool FINDMAX, bool EXACT>
-__global__ void __launch_bounds__(64)
+__global__ void __launch_bounds__(64, 2)
 k_irfft_score(const float* __restrict__ fold, uint64_t ntrials, WidthTable wt, uint32_t stride,
               float* __restrict__ scores, FilterOut fo) {
     using G = IrsGeom<NB>;
     extern __shared__ float lds[];
-    float* __restrict__ stage = lds;                  // [kTile]
-    float* __restrict__ prow  = lds + G::kTile;       // [64][stride]
-    auto* tw = reinterpret_cast<float2*>(prow + kWaveTrials * stride);  // [NB]
+    float* __restrict__ prow = lds;  // [64][stride]
+    auto* tw = reinterpret_cast<float2*>(prow + ((kWaveTrials * stride + 1) & ~1U));  // [NB]
     const int lane = static_cast<int>(threadIdx.x);
     const int mrow = lane & 15;   // A row / D column within the tile
     const int kq   = lane >> 4;   // A column / D row group
@@ -74,76 +113,97 @@ k_irfft_score(const float* __restrict__ fold, uint64_t ntrials, WidthTable wt, u
         tw[t] = make_float2(static_cast<float>(cs), static_cast<float>(sn));
     }
     wave_sync();
-    const uint64_t nfloats = ntrials * 2 * G::kRow;
-    const uint64_t ngroups = (ntrials + kWaveTrials - 1) / kWaveTrials;
-    constexpr int kLoads   = (G::kTile / 4 + 63) / 64;  // float4 loads per lane per tile
-    float4 pre[kLoads];
-    // loads of one tile (8 trials from trial c) into registers; zeros past the end
-    auto load_tile = [&](uint64_t c) {
-        const uint64_t base = c * 2 * G::kRow;  // 16-byte aligned: kTile % 4 == 0
+    // this lane's basis values, one register each (68 at 64 bins) for the whole
+    // kernel; opaque, or they would be formed again for every tile
+    float basis[G::kKs][G::kNt];
 #pragma unroll
-        for (int i = 0; i < kLoads; ++i) {
-            const int i4     = lane + 64 * i;
-            const uint64_t g = base + 4 * static_cast<uint64_t>(i4);
-            float4 v         = make_float4(0.0F, 0.0F, 0.0F, 0.0F);
-            if (i4 < G::kTile / 4) {
-                if (g + 4 <= nfloats) {
-                    v = *reinterpret_cast<const float4*>(fold + g);
-                } else {
-                    v.x = g + 0 < nfloats ? fold[g + 0] : 0.0F;
-                    v.y = g + 1 < nfloats ? fold[g + 1] : 0.0F;
-                    v.z = g + 2 < nfloats ? fold[g + 2] : 0.0F;
-                }
-            }
-            pre[i] = v;
+    for (int ks = 0; ks < G::kKs; ++ks) {
+#pragma unroll
+        for (int nt = 0; nt < G::kNt; ++nt) {
+            const int k   = ks + 1 == G::kKs ? NB + kq : 8 * (ks >> 1) + 2 * kq + (ks & 1);
+            basis[ks][nt] = irdft_basis<NB>(tw, k, 16 * nt + mrow);
+            asm volatile("" : "+v"(basis[ks][nt]));
         }
+    }
+    const uint64_t ngroups = (ntrials + kWaveTrials - 1) / kWaveTrials;
+    // A operands of one tile (8 trials from trial c), straight from the rows: K
+    // step 2i + j takes harmonic component 8i + 2 kq + j, so that a lane reads
+    // float2s; the last step is the real part of harmonic NB/2 in lane group 0.
+    // Zeros for trials past the end.
+    float2 pre[G::kF2];
+    float pre_last = 0.0F;
+    auto load_tile = [&](uint64_t c) {
+        const bool live = c + static_cast<uint64_t>(mrow >> 1) < ntrials;
+        const float* __restrict__ r =
+            fold + (live ? 2 * c + static_cast<uint64_t>(mrow) : 0) * G::kRow;
+#pragma unroll
+        for (int i = 0; i < G::kF2; ++i) {
+            const float2 v = *reinterpret_cast<const float2*>(r + 8 * i + 2 * kq);
+            pre[i].x       = live ? v.x : 0.0F;
+            pre[i].y       = live ? v.y : 0.0F;
+        }
+        const float v = r[NB];
+        pre_last      = live && kq == 0 ? v : 0.0F;
     };
+    load_tile(static_cast<uint64_t>(blockIdx.x) * kWaveTrials);
     for (uint64_t grp = blockIdx.x; grp < ngroups; grp += gridDim.x) {
         const uint64_t c0 = grp * kWaveTrials;
-        load_tile(c0);
 #pragma unroll 1
         for (int t = 0; t < kWaveTrials / kTileTrials; ++t) {
+            float a[G::kKs];
 #pragma unroll
-            for (int i = 0; i < kLoads; ++i) {
-                const int i4 = lane + 64 * i;
-                if (i4 < G::kTile / 4) {
-                    *reinterpret_cast<float4*>(stage + 4 * i4) = pre[i];
-                }
+            for (int i = 0; i < G::kF2; ++i) {
+                a[2 * i]     = pre[i].x;
+                a[2 * i + 1] = pre[i].y;
             }
-            wave_sync();
-            // prefetch this group's next tile while the matrix cores run
-            if (t + 1 < kWaveTrials / kTileTrials) {
-                load_tile(c0 + static_cast<uint64_t>(t + 1) * kTileTrials);
-            }
+            a[G::kKs - 1] = pre_last;
+            // the next tile, of this group or of the wave's next one, comes in
+            // while the matrix cores run and the widths are taken
+            load_tile(t + 1 < kWaveTrials / kTileTrials
+                          ? c0 + static_cast<uint64_t>(t + 1) * kTileTrials
+                          : c0 + static_cast<uint64_t>(gridDim.x) * kWaveTrials);
             f32x4 acc[G::kNt];
 #pragma unroll
             for (int nt = 0; nt < G::kNt; ++nt) {
                 acc[nt] = f32x4{0.0F, 0.0F, 0.0F, 0.0F};
             }
-            // an opaque zero keeps the basis reads inside the loop: hoisted, the 4 * kKs
-            // basis values would hold that many registers for the whole kernel
-            int zero = 0;
-            asm volatile("" : "+v"(zero));
 #pragma unroll
             for (int ks = 0; ks < G::kKs; ++ks) {
-                const int k   = 4 * ks + kq;
-                const float a = k < G::kRow ? stage[mrow * G::kRow + k] : 0.0F;
 #pragma unroll
                 for (int nt = 0; nt < G::kNt; ++nt) {
-                    const float b = irdft_basis<NB>(tw, k, 16 * nt + mrow, zero);
-                    acc[nt]       = __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, acc[nt], 0, 0, 0);
+                    acc[nt] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[ks], basis[ks][nt], acc[nt], 0,
+                                                                  0, 0);
                 }
             }
             // D rows 4*kq + v: trial 2*kq + v/2 of the tile, component v % 2
             const int tr = t * kTileTrials + 2 * kq;
+            float* __restrict__ prow0 = prow + tr * stride + mrow;
+            float* __restrict__ prow1 = prow0 + stride;
+            if constexpr (EXACT) {
+                // two accumulators at a time: one range check for the short
+                // correctly rounded sequences
 #pragma unroll
-            for (int nt = 0; nt < G::kNt; ++nt) {
-                const int bin = 16 * nt + mrow;
-                prow[tr * stride + bin]       = normalise<EXACT>(acc[nt][0], acc[nt][1]);
-                prow[(tr + 1) * stride + bin] = normalise<EXACT>(acc[nt][2], acc[nt][3]);
+                for (int nt = 0; nt < G::kNt; nt += 2) {
+                    const int nu   = nt + 1 < G::kNt ? nt + 1 : nt;
+                    const float4 p = normalise4_exact(
+                        make_float4(acc[nt][0], acc[nt][2], acc[nu][0], acc[nu][2]),
+                        make_float4(acc[nt][1], acc[nt][3], acc[nu][1], acc[nu][3]));
+                    prow0[16 * nt] = p.x;
+                    prow1[16 * nt] = p.y;
+                    if (nu != nt) {
+                        prow0[16 * nu] = p.z;
+                        prow1[16 * nu] = p.w;
+                    }
+                }
+            } else {
+#pragma unroll
+                for (int nt = 0; nt < G::kNt; ++nt) {
+                    prow0[16 * nt] = normalise<false>(acc[nt][0], acc[nt][1]);
+                    prow1[16 * nt] = normalise<false>(acc[nt][2], acc[nt][3]);
+                }
             }
-            wave_sync();  // the next tile overwrites the staged rows
         }
+        wave_sync();  // the rows are complete
         const uint64_t c = c0 + static_cast<uint64_t>(lane);
         if (c < ntrials) {
             float* __restrict__ row = prow + lane * stride;
@@ -155,23 +215,18 @@ k_irfft_score(const float* __restrict__ fold, uint64_t ntrials, WidthTable wt, u
                 ps[j] = acc;
             }
             const float sum = ps[NB - 1];
-#pragma unroll
-            for (int j = 0; j < NB; ++j) {
-                row[j] = ps[j];
-            }
-            // psum[i] for NB <= i < NB + w is psum[i - NB] + sum (the same FP32 add as a
-            // stored wrap extension), read through the power-of-two index mask
-            float best = -FLT_MAX;
+            float best      = -FLT_MAX;
             for (uint32_t iw = 0; iw < wt.n; ++iw) {
-                const uint32_t w = wt.w[iw];
-                float dmax       = -FLT_MAX;
+                // opaque once per width: otherwise the maxima of all NB - 1
+                // widths are formed ahead of the loop
 #pragma unroll
                 for (int j = 0; j < NB; ++j) {
-                    const uint32_t i = static_cast<uint32_t>(j) + w;
-                    float hv         = row[i & (NB - 1)];
-                    hv               = i >= static_cast<uint32_t>(NB) ? hv + sum : hv;
-                    dmax             = __builtin_fmaxf(dmax, hv - ps[j]);
+                    asm volatile("" : "+v"(ps[j]));
                 }
+                // every width's window with compile-time offsets, picked by a
+                // scalar branch on the wave-uniform width
+                const float dmax = window_max_reg<NB>(std::make_integer_sequence<int, NB - 1>{},
+                                                      ps, wt.w[iw]);
                 const float snr = ((wt.h[iw] + wt.b[iw]) * dmax) - (wt.b[iw] * sum);
                 if constexpr (FINDMAX) {
                     best = (best < snr) ? snr : best;
@@ -199,7 +254,7 @@ void launch_irs(const float2* fold, uint64_t ntrials, const WidthTable& wt, floa
                 const FilterOut& fo, hipStream_t s) {
     using G = IrsGeom<NB>;
     const uint32_t stride = NB + 1;  // odd: conflict-free per-lane rows
-    const size_t lds = (static_cast<size_t>(G::kTile) + kWaveTrials * stride + 2 * NB) *
+    const size_t lds = (((static_cast<size_t>(kWaveTrials) * stride + 1) & ~size_t{1}) + 2 * NB) *
                        sizeof(float);
     LOKI_REQUIRE(lds <= 65536, "irfft+score: LDS row too long");
     const uint64_t ngroups = (ntrials + kWaveTrials - 1) / kWaveTrials;

@@ -390,33 +390,43 @@ void* FFAExecutor::run_levels(const float* ts_e, const float* ts_v, void* buf_ev
             cp = m_ws->coords.as<FFACoord>() + off;
         }
     };
-    // Pass plan: levels l and l + 1 merged in one two-level pass where allowed
-    // (Fourier, or both stored in the tree's storage), pairing from the top down.
-    std::vector<uint8_t> two(last_level + 2, 0);  // two[l]: levels l, l+1 in one pass
+    // Pass plan, from the top down: span[l] levels from l on merged in one pass
+    // where allowed (Fourier: two or three; time: two, both stored in the tree's
+    // storage).
+    std::vector<uint8_t> span(last_level + 2, 1);
     SizeType passes = last_level;
+    // only where the tree does not grow: a pass whose output level is larger than
+    // its input level (the accel/jerk grid refining) gathers its input rows from a
+    // level a fraction of its size and measured slower than single passes
+    // (2^23-sample accel search, levels 10-11: 1.97 ms against 0.47 + 1.28 ms)
+    auto grows = [&](SizeType top, SizeType from) {
+        return m_plan.level_size(top) > m_plan.level_size(from) + m_plan.level_size(from) / 4;
+    };
     if (m_two_level && (m_fourier || kern::merge2_supported(static_cast<uint32_t>(nbins)))) {
         for (SizeType top = last_level; top >= 2;) {
-            const SizeType l     = top - 1;
-            const FoldStorage si = stored_as(l - 1, last_level, last_fp32);
-            const FoldStorage sb = stored_as(l, last_level, last_fp32);
-            const FoldStorage so = stored_as(top, last_level, last_fp32);
-            const bool to32      = last_fp32 && top == last_level;
-            // only where the tree does not grow: a pass whose output level is
-            // larger than its input level (the accel/jerk grid refining) gathers
-            // its four input rows from a level half its size and measured slower
-            // than two single passes (2^23-sample accel search, levels 10-11:
-            // 1.97 ms against 0.47 + 1.28 ms)
-            const bool grows = m_plan.level_size(top) > m_plan.level_size(l - 1) + m_plan.level_size(l - 1) / 4;
-            const bool storable =
-                m_fourier || (!to32 && sb == so &&
-                              (si == so || (si == FoldStorage::kF32 && so == FoldStorage::kBFP16)));
-            if (grows || !storable) {
+            SizeType n = 2;
+            if (m_fourier) {
+                if (top >= 3 && !grows(top, top - 3) && !grows(top, top - 2) &&
+                    kern::merge_fourier3_better(m_plan.ncoords()[top], m_plan.nsegments()[top],
+                                                static_cast<uint32_t>(nbins))) {
+                    n = 3;
+                }
+            } else {
+                const FoldStorage si = stored_as(top - 2, last_level, last_fp32);
+                const FoldStorage sb = stored_as(top - 1, last_level, last_fp32);
+                const FoldStorage so = stored_as(top, last_level, last_fp32);
+                if ((last_fp32 && top == last_level) || sb != so ||
+                    (si != so && !(si == FoldStorage::kF32 && so == FoldStorage::kBFP16))) {
+                    n = 1;
+                }
+            }
+            if (n == 1 || grows(top, top - 2)) {
                 top -= 1;  // this pair cannot be merged in one pass; try one lower
                 continue;
             }
-            two[l] = 1;
-            passes -= 1;
-            top -= 2;
+            span[top - n + 1] = static_cast<uint8_t>(n);
+            passes -= n - 1;
+            top -= n;
         }
     }
     void* const last = last_level % 2 == 0 ? buf_even : buf_odd;
@@ -427,54 +437,42 @@ void* FFAExecutor::run_levels(const float* ts_e, const float* ts_v, void* buf_ev
     }
     init_level(ts_e, ts_v, cur, other, last_fp32 && last_level == 0, s);
     for (SizeType l = 1; l <= last_level;) {
-        const FFACoord* cp      = nullptr;
-        const FFACoordFreq* cfp = nullptr;
-        tables(l, cp, cfp);
-        if (two[l] != 0) {
-            const FFACoord* cp2      = nullptr;
-            const FFACoordFreq* cfp2 = nullptr;
-            tables(l + 1, cp2, cfp2);
-            const int slot = m_timer.start(KernelKind::kMerge, static_cast<int>(l + 1), s);
-            if (m_fourier) {
-                kern::merge_fourier2(static_cast<const float2*>(cur), static_cast<float2*>(other),
-                                     cp, cfp, cp2, cfp2, m_plan.ncoords()[l + 1],
-                                     m_plan.ncoords()[l - 1], m_plan.nsegments()[l + 1],
-                                     static_cast<uint32_t>(nbins), s);
-            } else {
-                kern::merge_time2(cur, other, cp, cfp, cp2, cfp2, m_plan.ncoords()[l + 1],
-                                  m_plan.ncoords()[l], m_plan.ncoords()[l - 1],
-                                  m_plan.nsegments()[l + 1], m_plan.param_counts()[l + 1].back(),
-                                  static_cast<uint32_t>(nbins),
-                                  stored_as(l - 1, last_level, last_fp32),
-                                  stored_as(l + 1, last_level, last_fp32), 0.5F, s);
-            }
-            check_launch("two-level merge launch");
-            m_timer.stop(slot, s);
-            l += 2;
-        } else {
-            const int slot = m_timer.start(KernelKind::kMerge, static_cast<int>(l), s);
-            if (m_fourier) {
-                kern::merge_fourier(static_cast<const float2*>(cur), static_cast<float2*>(other),
-                                    cp, cfp, m_plan.ncoords()[l], m_plan.ncoords()[l - 1],
-                                    m_plan.nsegments()[l], static_cast<uint32_t>(nbins), s);
-            } else {
-                // FP16/BF16: (tail + head) * 0.5 keeps level l at 2^-(k0 + l); a last
-                // level returned in FP32 is unscaled by 2^(k0 + l - 1) instead.
-                // FP32 and block floating point are unscaled (scale unused).
-                const bool to32      = last_fp32 && l == last_level;
-                const FoldStorage si = stored_as(l - 1, last_level, last_fp32);
-                const FoldStorage so = stored_as(l, last_level, last_fp32);
-                const float scale =
-                    to32 ? std::ldexp(1.0F, m_k0 + static_cast<int>(l) - 1) : 0.5F;
-                kern::merge_time(cur, other, cp, cfp, m_plan.ncoords()[l],
-                                 m_plan.ncoords()[l - 1], m_plan.nsegments()[l],
-                                 m_plan.param_counts()[l].back(), static_cast<uint32_t>(nbins),
-                                 si, so, scale, s);
-            }
-            check_launch("merge launch");
-            m_timer.stop(slot, s);
-            l += 1;
+        const SizeType n   = span[l];
+        const SizeType top = l + n - 1;
+        const FFACoord* cp[kern::kFourierPassLevels]      = {};
+        const FFACoordFreq* cfp[kern::kFourierPassLevels] = {};
+        for (SizeType i = 0; i < n; ++i) {
+            tables(l + i, cp[i], cfp[i]);
         }
+        const int slot = m_timer.start(KernelKind::kMerge, static_cast<int>(top), s);
+        if (m_fourier) {
+            kern::merge_fourier(static_cast<const float2*>(cur), static_cast<float2*>(other),
+                                static_cast<uint32_t>(n), cp, cfp, m_plan.ncoords()[top],
+                                m_plan.ncoords()[l - 1], m_plan.nsegments()[top],
+                                static_cast<uint32_t>(nbins), s);
+        } else if (n == 2) {
+            kern::merge_time2(cur, other, cp[0], cfp[0], cp[1], cfp[1], m_plan.ncoords()[top],
+                              m_plan.ncoords()[l], m_plan.ncoords()[l - 1],
+                              m_plan.nsegments()[top], m_plan.param_counts()[top].back(),
+                              static_cast<uint32_t>(nbins),
+                              stored_as(l - 1, last_level, last_fp32),
+                              stored_as(top, last_level, last_fp32), 0.5F, s);
+        } else {
+            // FP16/BF16: (tail + head) * 0.5 keeps level l at 2^-(k0 + l); a last
+            // level returned in FP32 is unscaled by 2^(k0 + l - 1) instead.
+            // FP32 and block floating point are unscaled (scale unused).
+            const bool to32      = last_fp32 && l == last_level;
+            const FoldStorage si = stored_as(l - 1, last_level, last_fp32);
+            const FoldStorage so = stored_as(l, last_level, last_fp32);
+            const float scale    = to32 ? std::ldexp(1.0F, m_k0 + static_cast<int>(l) - 1) : 0.5F;
+            kern::merge_time(cur, other, cp[0], cfp[0], m_plan.ncoords()[l],
+                             m_plan.ncoords()[l - 1], m_plan.nsegments()[l],
+                             m_plan.param_counts()[l].back(), static_cast<uint32_t>(nbins), si,
+                             so, scale, s);
+        }
+        check_launch("merge launch");
+        m_timer.stop(slot, s);
+        l = top + 1;
         std::swap(cur, other);
     }
     LOKI_REQUIRE(cur == last, "merge passes: wrong landing buffer");

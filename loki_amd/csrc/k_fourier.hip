@@ -597,10 +597,9 @@ __device__ __forceinline__ uint32_t div_by(uint32_t n, const FastDiv& f) {
 struct FourierMergeArgs {
     const float2* in;
     float2* out;
-    const FFACoord* coords;         // poly levels
-    const FFACoordFreq* cf;         // freq-only levels
-    const FFACoord* coords_up;      // two levels: the upper level's records
-    const FFACoordFreq* cf_up;
+    // records of each level of the pass, the lowest first
+    const FFACoord* coords[kFourierPassLevels];   // poly levels
+    const FFACoordFreq* cf[kFourierPassLevels];   // freq-only levels
     uint64_t ncur, nprev, nseg;     // output level; input level's coordinates
     uint32_t nbf;
     FastDiv by_nbf, by_ncur;
@@ -655,16 +654,19 @@ __device__ __forceinline__ FFACoord record_of(const FFACoord* coords, const FFAC
 }
 
 // IDX: uint32_t when nseg * ncur * nbf < 2^32 (division by multiplication),
-// else uint64_t.  LEVELS 2: the output level's parents are formed from their
-// own parents (four rows) in registers and never stored.  SEGS: segments per
-// lane; their records, twiddles and row offsets are the same.  Consecutive
-// rows share parents and stay in one XCD's L2 (xcd_remap).  2^22 samples, 33
-// harmonics, 2.0 GB per level: one level 0.85 ms (0.90 before), two levels in
-// one pass 1.12 ms with four segments per lane, 1.31 ms with one, whose
-// VALU work (six twiddles per value, 1.0 ms) is then the bound.
+// else uint64_t.  LEVELS 2 and 3: the levels between are formed in registers
+// and never stored.  SEGS: segments per lane; their records, twiddles and row
+// offsets are the same.  Consecutive rows share parents and stay in one XCD's
+// L2 (xcd_remap).  2^22 samples, 33 harmonics, 2.0 GB per level: one level
+// 0.85 ms, two in one pass 1.12 ms with four segments per lane and 1.30 ms with
+// one (six twiddles per value, 1.0 ms of the vector unit), three in one pass
+// 1.73 ms with four (fourteen twiddles, eight gathered rows, 1.0 ms).  11 levels
+// as 2 + 3 + 3 + 3: 6.49 ms, as 2 + 2 + 2 + 2 + 2 + 1: 6.61 ms.
 template <int LEVELS, int SEGS, bool POLY, bool POW2, typename IDX>
 __global__ void __launch_bounds__(kBlock)
 k_merge_fourier(FourierMergeArgs a) {
+    constexpr int kRows  = 1 << LEVELS;  // input rows of one output row
+    constexpr int kNodes = kRows - 1;    // output row and the rows between, as a heap
     const IDX ncur  = static_cast<IDX>(a.ncur);
     const IDX total = static_cast<IDX>(a.nseg / SEGS) * ncur * a.nbf;
     for (IDX t = static_cast<IDX>(xcd_remap(blockIdx.x, gridDim.x)) * kBlock + threadIdx.x;
@@ -683,45 +685,49 @@ k_merge_fourier(FourierMergeArgs a) {
         const auto kf      = static_cast<float>(k);
         const uint64_t row = 2ULL * a.nbf;  // complex values per row
         float2* w          = a.out + (seg * a.ncur + c) * row + k;
-        if constexpr (LEVELS == 1) {
-            const FFACoord cd    = record_of<POLY>(a.coords, a.cf, c);
-            const TwiddlePair tw = twiddle_pair<POLY, POW2>(a, cd, kf);
-            const float2* pt     = a.in + ((2 * seg) * a.nprev + cd.i_tail) * row + k;
-            const float2* ph     = a.in + ((2 * seg + 1) * a.nprev + cd.i_head) * row + k;
+        // node i's children are 2i + 1 (tail, earlier half) and 2i + 2 (head);
+        // the nodes after the last level's are the input rows, in segment order
+        FFACoord node[kNodes];
+        TwiddlePair tw[kNodes];
+        const float2* p[kRows];
+        node[0] = record_of<POLY>(a.coords[LEVELS - 1], a.cf[LEVELS - 1], c);
 #pragma unroll
-            for (int i = 0; i < SEGS; ++i) {
-                const FourierPair o =
-                    merge_pair<POLY>(load_pair(pt, a.nbf), load_pair(ph, a.nbf), tw);
-                w[0]     = o.e;
-                w[a.nbf] = o.v;
-                pt += 2 * a.nprev * row;
-                ph += 2 * a.nprev * row;
-                w += a.ncur * row;
-            }
-        } else {
-            const FFACoord up    = record_of<POLY>(a.coords_up, a.cf_up, c);
-            const FFACoord lt    = record_of<POLY>(a.coords, a.cf, up.i_tail);
-            const FFACoord lh    = record_of<POLY>(a.coords, a.cf, up.i_head);
-            const TwiddlePair tt = twiddle_pair<POLY, POW2>(a, lt, kf);
-            const TwiddlePair th = twiddle_pair<POLY, POW2>(a, lh, kf);
-            const TwiddlePair tu = twiddle_pair<POLY, POW2>(a, up, kf);
-            const float2* base   = a.in + seg * 4 * a.nprev * row + k;
-            const float2* p0     = base + lt.i_tail * row;
-            const float2* p1     = base + (a.nprev + lt.i_head) * row;
-            const float2* p2     = base + (2 * a.nprev + lh.i_tail) * row;
-            const float2* p3     = base + (3 * a.nprev + lh.i_head) * row;
+        for (int d = 1; d < LEVELS; ++d) {
 #pragma unroll
-            for (int i = 0; i < SEGS; ++i) {
-                const uint64_t off   = static_cast<uint64_t>(i) * 4 * a.nprev * row;
-                const FourierPair mt = merge_pair<POLY>(load_pair(p0 + off, a.nbf),
-                                                        load_pair(p1 + off, a.nbf), tt);
-                const FourierPair mh = merge_pair<POLY>(load_pair(p2 + off, a.nbf),
-                                                        load_pair(p3 + off, a.nbf), th);
-                const FourierPair o  = merge_pair<POLY>(mt, mh, tu);
-                w[0]                 = o.e;
-                w[a.nbf]             = o.v;
-                w += a.ncur * row;
+            for (int i = (1 << d) - 1; i < (2 << d) - 1; ++i) {
+                const FFACoord& up = node[(i - 1) / 2];
+                node[i] = record_of<POLY>(a.coords[LEVELS - 1 - d], a.cf[LEVELS - 1 - d],
+                                          (i & 1) != 0 ? up.i_tail : up.i_head);
             }
+        }
+#pragma unroll
+        for (int i = 0; i < kNodes; ++i) {
+            tw[i] = twiddle_pair<POLY, POW2>(a, node[i], kf);
+        }
+        const float2* base = a.in + seg * kRows * a.nprev * row + k;
+#pragma unroll
+        for (int i = 0; i < kRows; ++i) {
+            const FFACoord& up = node[kRows / 2 - 1 + i / 2];
+            p[i] = base + (i * a.nprev + ((i & 1) == 0 ? up.i_tail : up.i_head)) * row;
+        }
+#pragma unroll
+        for (int sgi = 0; sgi < SEGS; ++sgi) {
+            const uint64_t off = static_cast<uint64_t>(sgi) * kRows * a.nprev * row;
+            FourierPair v[kRows];
+#pragma unroll
+            for (int i = 0; i < kRows; ++i) {
+                v[i] = load_pair(p[i] + off, a.nbf);
+            }
+#pragma unroll
+            for (int d = LEVELS - 1; d >= 0; --d) {
+#pragma unroll
+                for (int i = 0; i < (1 << d); ++i) {
+                    v[i] = merge_pair<POLY>(v[2 * i], v[2 * i + 1], tw[(1 << d) - 1 + i]);
+                }
+            }
+            w[0]     = v[0].e;
+            w[a.nbf] = v[0].v;
+            w += a.ncur * row;
         }
     }
 }
@@ -858,21 +864,26 @@ void launch_merge_fourier_segs(const FourierMergeArgs& a, bool pow2, unsigned g,
     }
 }
 
+// Segments per lane: 4 while that leaves 16 waves per SIMD's worth of lanes, 2
+// while it leaves as many.
+constexpr uint64_t kSegLanes = 1ULL << 20;
+
+/// Whether 32 bits index total values; the grid-stride loop must not overflow.
+bool narrow_index(uint64_t total) {
+    return total + static_cast<uint64_t>(grid_for(total)) * kBlock < (1ULL << 32);
+}
+
 template <int LEVELS, bool POLY>
 void launch_merge_fourier(const FourierMergeArgs& a, bool pow2, hipStream_t s) {
     const uint64_t total = a.nseg * a.ncur * a.nbf;
-    // the grid-stride loop must not overflow the index type
-    const bool narrow =
-        total + static_cast<uint64_t>(grid_for(total)) * kBlock < (1ULL << 32) &&
-        a.ncur < (1ULL << 32);
-    // Segments per lane: 4 while that leaves 16 waves per SIMD's worth of lanes
-    // (2^20), 2 while it leaves as many.
-    constexpr uint64_t kLanes = 1ULL << 20;
-    if (!narrow) {
-        launch_merge_fourier_segs<LEVELS, 1, POLY, uint64_t>(a, pow2, grid_for(total), s);
-    } else if (a.nseg % 4 == 0 && total / 4 >= kLanes) {
+    [[maybe_unused]] const bool narrow = narrow_index(total) && a.ncur < (1ULL << 32);
+    if constexpr (LEVELS == 3) {  // merge_fourier3_better holds
         launch_merge_fourier_segs<LEVELS, 4, POLY, uint32_t>(a, pow2, grid_for(total / 4), s);
-    } else if (a.nseg % 2 == 0 && total / 2 >= kLanes) {
+    } else if (!narrow) {
+        launch_merge_fourier_segs<LEVELS, 1, POLY, uint64_t>(a, pow2, grid_for(total), s);
+    } else if (a.nseg % 4 == 0 && total / 4 >= kSegLanes) {
+        launch_merge_fourier_segs<LEVELS, 4, POLY, uint32_t>(a, pow2, grid_for(total / 4), s);
+    } else if (a.nseg % 2 == 0 && total / 2 >= kSegLanes) {
         launch_merge_fourier_segs<LEVELS, 2, POLY, uint32_t>(a, pow2, grid_for(total / 2), s);
     } else {
         launch_merge_fourier_segs<LEVELS, 1, POLY, uint32_t>(a, pow2, grid_for(total), s);
@@ -898,46 +909,36 @@ FourierMergeArgs fourier_merge_args(const float2* in, float2* out, uint64_t ncur
 
 }  // namespace
 
-void merge_fourier(const float2* in, float2* out, const FFACoord* coords,
-                   const FFACoordFreq* coords_freq, uint64_t ncur, uint64_t nprev, uint64_t nseg,
-                   uint32_t nbins, hipStream_t s) {
-    LOKI_REQUIRE((coords == nullptr) != (coords_freq == nullptr),
-                 "merge: exactly one coordinate table");
-    if (ncur == 0 || nseg == 0) {
-        return;
-    }
-    auto a              = fourier_merge_args(in, out, ncur, nprev, nseg, nbins);
-    a.coords            = coords;
-    a.cf                = coords_freq;
-    const bool pow2     = (nbins & (nbins - 1)) == 0;
-    if (coords != nullptr) {
-        launch_merge_fourier<1, true>(a, pow2, s);
-    } else {
-        launch_merge_fourier<1, false>(a, pow2, s);
-    }
+bool merge_fourier3_better(uint64_t ncur, uint64_t nseg, uint32_t nbins) {
+    const uint64_t total = nseg * ncur * (nbins / 2 + 1);
+    return nseg % 4 == 0 && total / 4 >= kSegLanes && narrow_index(total);
 }
 
-void merge_fourier2(const float2* in, float2* out, const FFACoord* coords,
-                    const FFACoordFreq* coords_freq, const FFACoord* coords_up,
-                    const FFACoordFreq* coords_freq_up, uint64_t ncur, uint64_t nprev,
-                    uint64_t nseg, uint32_t nbins, hipStream_t s) {
-    LOKI_REQUIRE((coords == nullptr) != (coords_freq == nullptr) &&
-                     (coords == nullptr) == (coords_up == nullptr) &&
-                     (coords_freq == nullptr) == (coords_freq_up == nullptr),
-                 "merge: exactly one coordinate table per level");
+void merge_fourier(const float2* in, float2* out, uint32_t levels, const FFACoord* const* coords,
+                   const FFACoordFreq* const* coords_freq, uint64_t ncur, uint64_t nprev,
+                   uint64_t nseg, uint32_t nbins, hipStream_t s) {
+    LOKI_REQUIRE(levels >= 1 && levels <= kFourierPassLevels, "merge: levels out of range");
+    auto a = fourier_merge_args(in, out, ncur, nprev, nseg, nbins);
+    for (uint32_t l = 0; l < levels; ++l) {
+        a.coords[l] = coords[l];
+        a.cf[l]     = coords_freq[l];
+        LOKI_REQUIRE((a.coords[l] == nullptr) != (a.cf[l] == nullptr) &&
+                         (a.coords[l] == nullptr) == (a.coords[0] == nullptr),
+                     "merge: exactly one coordinate table per level");
+    }
     if (ncur == 0 || nseg == 0) {
         return;
     }
-    auto a              = fourier_merge_args(in, out, ncur, nprev, nseg, nbins);
-    a.coords            = coords;
-    a.cf                = coords_freq;
-    a.coords_up         = coords_up;
-    a.cf_up             = coords_freq_up;
-    const bool pow2     = (nbins & (nbins - 1)) == 0;
-    if (coords != nullptr) {
-        launch_merge_fourier<2, true>(a, pow2, s);
+    const bool pow2 = (nbins & (nbins - 1)) == 0;
+    const bool poly = a.coords[0] != nullptr;
+    LOKI_REQUIRE(levels < 3 || merge_fourier3_better(ncur, nseg, nbins),
+                 "merge: three levels need four segments per lane");
+    if (levels == 1) {
+        poly ? launch_merge_fourier<1, true>(a, pow2, s) : launch_merge_fourier<1, false>(a, pow2, s);
+    } else if (levels == 2) {
+        poly ? launch_merge_fourier<2, true>(a, pow2, s) : launch_merge_fourier<2, false>(a, pow2, s);
     } else {
-        launch_merge_fourier<2, false>(a, pow2, s);
+        poly ? launch_merge_fourier<3, true>(a, pow2, s) : launch_merge_fourier<3, false>(a, pow2, s);
     }
 }
 

@@ -152,19 +152,24 @@ void brute_fold_spectra(const float* ts_e, const float* ts_v, uint64_t nseg, uin
                         const double* freqs_dev, uint32_t nfreqs, uint32_t nbins, double tsamp,
                         double t_ref, float2* fold, void* spec, hipStream_t s);
 
-/// Fourier-domain merge of one level (freq-only when coords_freq != nullptr):
-/// phase rotation by the fractional shifts, rows of [2, nbins/2+1] float2.
-void merge_fourier(const float2* in, float2* out, const FFACoord* coords,
-                   const FFACoordFreq* coords_freq, uint64_t ncur, uint64_t nprev, uint64_t nseg,
-                   uint32_t nbins, hipStream_t s);
+/// Most levels that one Fourier merge pass takes.
+constexpr uint32_t kFourierPassLevels = 3;
 
-/// Two levels in one pass, the same values as two merge_fourier calls: coords
-/// of the lower level, coords_up of the upper (output) level, ncur its
-/// coordinates and nseg its segments, nprev the input level's coordinates.
-void merge_fourier2(const float2* in, float2* out, const FFACoord* coords,
-                    const FFACoordFreq* coords_freq, const FFACoord* coords_up,
-                    const FFACoordFreq* coords_freq_up, uint64_t ncur, uint64_t nprev,
-                    uint64_t nseg, uint32_t nbins, hipStream_t s);
+/// Fourier-domain merge of `levels` (1 to kFourierPassLevels) levels in one pass
+/// (freq-only when coords_freq[l] != nullptr): phase rotation by the fractional
+/// shifts, rows of [2, nbins/2+1] float2; the same values as one pass per level.
+/// coords / coords_freq: each level's table, the lowest first; ncur and nseg:
+/// coordinates and segments of the output level; nprev: the input level's
+/// coordinates.
+void merge_fourier(const float2* in, float2* out, uint32_t levels, const FFACoord* const* coords,
+                   const FFACoordFreq* const* coords_freq, uint64_t ncur, uint64_t nprev,
+                   uint64_t nseg, uint32_t nbins, hipStream_t s);
+
+/// Whether a pass with this output level should take three levels (required
+/// of such a pass): four segments per lane share the twiddles of its seven merges
+/// and still fill the card.  With one segment per lane a pass is bound by forming
+/// them (2^19 samples of 50 bins: 108 us for the fold, 100 us in passes of two).
+bool merge_fourier3_better(uint64_t ncur, uint64_t nseg, uint32_t nbins);
 
 /// Inverse real DFT of nrows rows of nbins/2+1 float2 into rows of nbins
 /// floats, scaled by 1/nbins (C2R + normalisation).

@@ -230,7 +230,8 @@ int loki_ffa_set_two_level_merges(loki_ffa_t ffa, int enable);
  * (|dS/N| ~ 1e-6, the analogue of the reference CUDA path's fast-math e/sqrtf(v),
  * score_cuda.cu:82).  No reference counterpart as a switch. */
 int loki_ffa_set_exact_norm(loki_ffa_t ffa, int exact);
-/* Fourier brute fold precision: 0 (default) FP32 matrix cores; 1 bf16 matrix cores with each
+/* Fourier brute fold precision: 0 (default) FP32 (chunk spectra, or FP32 matrix
+ * cores where they are faster); 1 bf16 matrix cores with each
  * operand split into high and low bf16 parts (three products per term, FP32 accumulation,
  * ~2^-17 relative per product) for nbins <= 129.  No reference counterpart (the reference's
  * Fourier brute fold is FP32, kernels_cuda.cu:780-965). */

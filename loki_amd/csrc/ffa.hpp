@@ -145,7 +145,7 @@ public:
     /// CPU's correctly rounded e * (1/sqrt(v))) or the hardware rsqrt.
     void set_exact_norm(bool on) noexcept { m_exact_norm = on; }
     /// Fourier brute fold on bf16 matrix cores with split (high + low) bf16
-    /// operands and FP32 accumulation instead of FP32 matrix cores (default
+    /// operands and FP32 accumulation instead of the FP32 path (default
     /// off; nbins <= 129, else FP32).
     void set_dft_split_bf16(bool on) noexcept { m_dft_split = on; }
     /// Storage precision of fold levels 0..L-2 (time domain only); the final

@@ -121,7 +121,8 @@ void merge_time(const void* in, void* out, const FFACoord* coords,
 
 /// Fourier brute fold: fold [nseg, nfreqs, 2, nbins/2+1] complex (float2) of
 /// exp(-2 pi i m f (k tsamp - t_ref)) sums; FP32 matrix-core DFT with FP64
-/// phases, harmonic 0 by FP64 reduction.  nbins in [2, 256].
+/// phases, harmonic 0 by FP64 reduction.  nbins in [2, 256].  For short segments
+/// or few frequencies; otherwise brute_fold_spectra is faster.
 /// split_bf16: harmonics on bf16 matrix cores with each operand split into
 /// high and low bf16 parts (three products per term, FP32 accumulation) for
 /// nbins <= 129; otherwise FP32 matrix cores.

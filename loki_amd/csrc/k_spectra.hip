@@ -220,6 +220,8 @@ constexpr int kFoldThreads = 512;
 // points of 16 bytes per value of both series.
 // TURN: the chunk's centre is not at t_ref (or there are several chunks), and
 // each value is turned by the phase of its chunk's centre.
+// Harmonic 0 is the segment's plain sum, the same for every frequency: the
+// chunks' FP64 sums are added in FP64 and rounded once.
 template <int OUTS, bool TURN>
 __global__ void __launch_bounds__(kFoldThreads)
 k_spectra_fold(SpecFoldArgs a) {
@@ -252,6 +254,7 @@ k_spectra_fold(SpecFoldArgs a) {
         for (int o = 0; o < OUTS; ++o) {
             acc[o] = make_float4(0.0F, 0.0F, 0.0F, 0.0F);
         }
+        double2 dc = make_double2(0.0, 0.0);
         for (uint32_t c = 0; c < a.nchunk; ++c) {
             __syncthreads();  // the previous chunk's readers are done
             const float4* src = a.spec + (seg * a.nchunk + c) * npt;
@@ -259,7 +262,9 @@ k_spectra_fold(SpecFoldArgs a) {
                 sp[i] = src[i];
             }
             __syncthreads();
-            const double2 dc = *reinterpret_cast<const double2*>(sp + (npt - 1));
+            const double2 sums = *reinterpret_cast<const double2*>(sp + (npt - 1));
+            dc.x += sums.x;
+            dc.y += sums.y;
 #pragma unroll
             for (int o = 0; o < OUTS; ++o) {
                 float4 v = spec_value(sp + first[o], w[o]);
@@ -271,9 +276,6 @@ k_spectra_fold(SpecFoldArgs a) {
                     const float2 z  = turns((ph - floor(ph)) * static_cast<double>(hm[o]));
                     v = make_float4(fmaf(v.x, z.x, -(v.y * z.y)), fmaf(v.x, z.y, v.y * z.x),
                                     fmaf(v.z, z.x, -(v.w * z.y)), fmaf(v.z, z.y, v.w * z.x));
-                }
-                if (hm[o] == 0) {  // the segment sum itself
-                    v = make_float4(static_cast<float>(dc.x), 0.0F, static_cast<float>(dc.y), 0.0F);
                 }
                 if constexpr (TURN) {
                     acc[o].x += v.x;
@@ -287,6 +289,9 @@ k_spectra_fold(SpecFoldArgs a) {
         }
 #pragma unroll
         for (int o = 0; o < OUTS; ++o) {
+            if (hm[o] == 0) {
+                acc[o] = make_float4(static_cast<float>(dc.x), 0.0F, static_cast<float>(dc.y), 0.0F);
+            }
             if (valid[o]) {
                 float2* row = a.fold + ((seg * a.nfreqs + fi[o]) * 2) * a.nbf + hm[o];
                 row[0]      = make_float2(acc[o].x, acc[o].y);

@@ -60,6 +60,32 @@ def test_fold_from_spectra_within_bound(oracle, seglen, nseg, nbins, nfreqs, t_r
     assert np.all(got[..., 0].imag == 0)
 
 
+@pytest.mark.parametrize(("seglen", "nseg", "nfreqs", "t_ref"), [
+    (2048, 3, 50, 0.0),          # one chunk
+    (2049, 5, 64, 0.0),          # two, the second of one sample
+    (65536, 4, 51, 1.7),         # 32
+    (1 << 20, 2, 3, 0.0),        # 512
+])
+def test_harmonic_zero_is_rounded_once(seglen, nseg, nfreqs, t_ref):
+    """Harmonic 0 is the segment's sum in FP64, rounded once to FP32: within u = 2^-24 of it
+    and the FP64 sum's own error, at most seglen 2^-53 of the L1 norm."""
+    from loki_amd import libculoki
+
+    rng = np.random.default_rng(seglen)
+    n = seglen * nseg
+    ts_e = (3.0 + rng.standard_normal(n)).astype(np.float32)
+    ts_v = (1000.0 + 20.0 * rng.standard_normal(n)).astype(np.float32)
+    freqs = np.linspace(0.7, 90.0, nfreqs)
+    got = libculoki.fold.compute_brute_fold_fourier_cuda(ts_e, ts_v, freqs, seglen, 16, TSAMP,
+                                                         t_ref).reshape(nseg, nfreqs, 2, 9)
+    x = np.stack([ts_e.reshape(nseg, seglen), ts_v.reshape(nseg, seglen)], 1).astype(np.longdouble)
+    want = x.sum(axis=2).astype(np.float64)[:, None]
+    l1 = np.abs(x).sum(axis=2).astype(np.float64)[:, None]
+    err = np.abs(got[..., 0].real.astype(np.float64) - want)
+    assert np.all(err <= U * np.abs(want) + seglen * 2.0**-53 * l1), float((err / want).max() / U)
+    assert np.all(got[..., 0].imag == 0)
+
+
 def test_series_do_not_mix():
     """A NaN in ts_e stays out of the variance rows and of the other segments, and variances
     twelve decades above the samples leave them exact."""

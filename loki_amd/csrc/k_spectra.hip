@@ -226,6 +226,7 @@ template <int OUTS, bool TURN>
 __global__ void __launch_bounds__(kFoldThreads)
 k_spectra_fold(SpecFoldArgs a) {
     extern __shared__ float4 sp[];
+    __shared__ double s_dc[2];  // FP64 registers for it would cost a workgroup per CU
     const uint32_t blk  = xcd_remap(blockIdx.x, gridDim.x);
     const uint32_t ob   = blk % a.nblk_out;
     const uint64_t seg0 = static_cast<uint64_t>(blk / a.nblk_out) * a.segs_per_block;
@@ -254,7 +255,6 @@ k_spectra_fold(SpecFoldArgs a) {
         for (int o = 0; o < OUTS; ++o) {
             acc[o] = make_float4(0.0F, 0.0F, 0.0F, 0.0F);
         }
-        double2 dc = make_double2(0.0, 0.0);
         for (uint32_t c = 0; c < a.nchunk; ++c) {
             __syncthreads();  // the previous chunk's readers are done
             const float4* src = a.spec + (seg * a.nchunk + c) * npt;
@@ -262,9 +262,10 @@ k_spectra_fold(SpecFoldArgs a) {
                 sp[i] = src[i];
             }
             __syncthreads();
-            const double2 sums = *reinterpret_cast<const double2*>(sp + (npt - 1));
-            dc.x += sums.x;
-            dc.y += sums.y;
+            if (threadIdx.x < 2) {
+                const double x     = reinterpret_cast<const double*>(sp + (npt - 1))[threadIdx.x];
+                s_dc[threadIdx.x] = c == 0 ? x : s_dc[threadIdx.x] + x;
+            }
 #pragma unroll
             for (int o = 0; o < OUTS; ++o) {
                 float4 v = spec_value(sp + first[o], w[o]);
@@ -287,10 +288,13 @@ k_spectra_fold(SpecFoldArgs a) {
                 }
             }
         }
+        __syncthreads();  // s_dc is complete
+        const auto dc_e = static_cast<float>(s_dc[0]);
+        const auto dc_v = static_cast<float>(s_dc[1]);
 #pragma unroll
         for (int o = 0; o < OUTS; ++o) {
             if (hm[o] == 0) {
-                acc[o] = make_float4(static_cast<float>(dc.x), 0.0F, static_cast<float>(dc.y), 0.0F);
+                acc[o] = make_float4(dc_e, 0.0F, dc_v, 0.0F);
             }
             if (valid[o]) {
                 float2* row = a.fold + ((seg * a.nfreqs + fi[o]) * 2) * a.nbf + hm[o];

@@ -160,7 +160,9 @@ int loki_ffa_create(loki_config_t cfg, int fold_type, int device_id, loki_ffa_t*
  * (ffa.hpp:100-153): FFAs made with one workspace share its device buffers (the ping-pong
  * partner fold, the second scores buffer and the shift tables), each growing them to its plan,
  * so many plans (the chunks of a frequency sweep) hold one set of buffers sized by the largest.
- * They must not run concurrently.  buffer_bytes / coord_bytes (0: none) preallocate.  The
+ * They must not run concurrently.  buffer_bytes / coord_bytes (0: none) preallocate.  A
+ * Fourier FFA forms its chunk spectra (16 to 34 bytes per sample) in the ping-pong partner; one
+ * whose level buffers are smaller than min(spectra, 256 MiB) keeps that much more.  The
  * workspace lives until it and every FFA made with it are destroyed. */
 typedef struct loki_ffa_workspace_s* loki_ffa_workspace_t;
 int loki_ffa_workspace_create(int device_id, size_t buffer_bytes, size_t coord_bytes,
@@ -469,7 +471,8 @@ int loki_brute_fold_time_device_noalloc(const float* ts_e, const float* ts_v, si
 
 /* compute_brute_fold_cuda<ComplexTypeCUDA> (fold_cuda.cu:260-277, kernels_cuda.cu:1012-1061):
  * fold has (nsamps/segment_len) * nfreqs * 2 * (nbins/2+1) complex64 values
- * (interleaved float pairs); nbins in [2, 256]. */
+ * (interleaved float pairs); nbins in [2, 256].  The call allocates and frees the frequencies
+ * and up to 64 MiB (or one segment's chunk spectra, 16 to 34 bytes per sample). */
 int loki_brute_fold_fourier_host(const float* ts_e, const float* ts_v, size_t nsamps,
                                  const double* freqs, size_t nfreqs, size_t segment_len,
                                  size_t nbins, double tsamp, double t_ref, float* fold,

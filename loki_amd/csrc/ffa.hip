@@ -341,10 +341,20 @@ void FFAExecutor::init_level(const float* ts_e, const float* ts_v, void* out, vo
         const auto nfreqs  = static_cast<uint32_t>(m_plan.param_counts()[0].back());
         const auto nb      = static_cast<uint32_t>(nbins);
         if (!m_dft_split && kern::spectra_fold_better(seglen, nfreqs)) {
-            m_ws->spectra.reserve(kern::spectra_bytes(nseg, seglen));
+            // The spectra go into the partner buffer (buffer_size elements), free until
+            // the first merge.  Only a plan whose levels are smaller than they are (few
+            // frequencies of long segments) keeps a buffer for them.
+            const SizeType bytes = kern::spectra_bytes(nseg, seglen, kern::kMaxSpectra);
+            const auto base      = reinterpret_cast<uintptr_t>(scratch);
+            const auto at        = (base + 15) & ~uintptr_t{15};
+            auto* spec           = reinterpret_cast<void*>(at);
+            if (at + bytes > base + m_plan.buffer_size() * elem_bytes()) {
+                m_ws->spectra.reserve(bytes);
+                spec = m_ws->spectra.get();
+            }
             kern::brute_fold_spectra(ts_e, ts_v, nseg, seglen, m_bf_freqs.as<double>(), nfreqs, nb,
                                      m_plan.config().get_tsamp(), t_ref,
-                                     static_cast<float2*>(out), m_ws->spectra.get(), s);
+                                     static_cast<float2*>(out), spec, bytes, s);
         } else {
             kern::brute_fold_fourier(ts_e, ts_v, nseg, seglen, m_bf_freqs.as<double>(), nfreqs, nb,
                                      m_plan.config().get_tsamp(), t_ref,
@@ -825,22 +835,25 @@ void brute_fold_fourier_device(const float* ts_e, const float* ts_v, SizeType ns
     LOKI_REQUIRE(nbins >= 2 && nbins <= 256, "BruteFold: Fourier fold needs nbins in [2, 256]");
     LOKI_REQUIRE(segment_len < (1ULL << 32) && freqs.size() < (1ULL << 32),
                  "BruteFold: segment too long");
-    DeviceBuffer d_freqs(freqs.size() * sizeof(double));
-    hip_check(hipMemcpyAsync(d_freqs.get(), freqs.data(), freqs.size() * sizeof(double),
+    const auto seglen  = static_cast<uint32_t>(segment_len);
+    const auto nfreqs  = static_cast<uint32_t>(freqs.size());
+    const auto nb      = static_cast<uint32_t>(nbins);
+    const SizeType ns  = nsamps / segment_len;
+    const bool spectra = kern::spectra_fold_better(seglen, nfreqs);
+    // one allocation: the spectra (16-byte aligned), then the frequencies
+    const SizeType spec_bytes =
+        spectra ? kern::spectra_bytes(ns, seglen, kern::kMaxSpectraOneOff) : 0;
+    DeviceBuffer buf(spec_bytes + freqs.size() * sizeof(double));
+    auto* d_freqs = reinterpret_cast<double*>(static_cast<char*>(buf.get()) + spec_bytes);
+    hip_check(hipMemcpyAsync(d_freqs, freqs.data(), freqs.size() * sizeof(double),
                              hipMemcpyHostToDevice, s),
               "copy frequencies");
-    const auto seglen = static_cast<uint32_t>(segment_len);
-    const auto nfreqs = static_cast<uint32_t>(freqs.size());
-    const auto nb     = static_cast<uint32_t>(nbins);
-    const SizeType ns = nsamps / segment_len;
-    DeviceBuffer d_spec;
-    if (kern::spectra_fold_better(seglen, nfreqs)) {
-        d_spec.reserve(kern::spectra_bytes(ns, seglen));
-        kern::brute_fold_spectra(ts_e, ts_v, ns, seglen, d_freqs.as<double>(), nfreqs, nb, tsamp,
-                                 t_ref, fold, d_spec.get(), s);
+    if (spectra) {
+        kern::brute_fold_spectra(ts_e, ts_v, ns, seglen, d_freqs, nfreqs, nb, tsamp, t_ref, fold,
+                                 buf.get(), spec_bytes, s);
     } else {
-        kern::brute_fold_fourier(ts_e, ts_v, ns, seglen, d_freqs.as<double>(), nfreqs, nb, tsamp,
-                                 t_ref, fold, s);
+        kern::brute_fold_fourier(ts_e, ts_v, ns, seglen, d_freqs, nfreqs, nb, tsamp, t_ref, fold,
+                                 s);
     }
     check_launch("Fourier brute fold launch");
     // The frequencies and spectra are freed on return: finish before that.

@@ -64,8 +64,7 @@ private:
 };
 
 /// Device buffers an FFA borrows (workspace.hpp:169-206 FFAWorkspaceCUDA): the
-/// ping-pong partner, the second scores buffer, the shift tables and the chunk
-/// spectra.  FFAs
+/// ping-pong partner, the second scores buffer and the shift tables.  FFAs
 /// that share one run one at a time; each grows the buffers to its plan.
 /// Uses on different streams are ordered: a use on stream s first waits for
 /// an event recorded at the end of the previous use on another stream.
@@ -78,7 +77,9 @@ struct FFAWorkspace {
     DeviceBuffer internal;
     DeviceBuffer result;
     DeviceBuffer coords;
-    DeviceBuffer spectra;  ///< chunk spectra of the Fourier brute fold
+    /// chunk spectra of a Fourier brute fold that do not fit the partner buffer:
+    /// at most kern::kMaxSpectra, or one segment's
+    DeviceBuffer spectra;
 
     /// Before enqueueing work that touches the buffers on `s`.
     void begin_use(hipStream_t s);
@@ -235,7 +236,8 @@ void brute_fold_time_device(const float* ts_e, const float* ts_v, SizeType nsamp
                             std::span<const double> freqs, SizeType segment_len, SizeType nbins,
                             double tsamp, double t_ref, float* fold, hipStream_t s);
 /// Standalone Fourier brute fold: fold has nsamps/segment_len * nfreqs * 2 *
-/// (nbins/2+1) float2 elements.  Synchronises `s`.
+/// (nbins/2+1) float2 elements.  Allocates its workspace (at most
+/// kern::kMaxSpectraOneOff or one segment's spectra) and synchronises `s`.
 void brute_fold_fourier_device(const float* ts_e, const float* ts_v, SizeType nsamps,
                                std::span<const double> freqs, SizeType segment_len,
                                SizeType nbins, double tsamp, double t_ref, float2* fold,

@@ -341,9 +341,19 @@ SpectraShape spectra_shape(uint64_t seglen) {
     return sh;
 }
 
-uint64_t spectra_bytes(uint64_t nseg, uint64_t seglen) {
+namespace {
+
+/// Bytes of one segment's spectra.
+uint64_t segment_bytes(uint64_t seglen) {
     const auto sh = spectra_shape(seglen);
-    return nseg * sh.nchunk * spec_stride(sh.m) * sizeof(float4);
+    return sh.nchunk * spec_stride(sh.m) * sizeof(float4);
+}
+
+}  // namespace
+
+uint64_t spectra_bytes(uint64_t nseg, uint64_t seglen, uint64_t max_bytes) {
+    const uint64_t one = segment_bytes(seglen);
+    return std::min(nseg, std::max<uint64_t>(max_bytes / one, 1)) * one;
 }
 
 void chunk_spectra(const float* ts_e, const float* ts_v, uint64_t nseg, uint64_t seglen,
@@ -376,19 +386,21 @@ bool spectra_fold_better(uint32_t seglen, uint32_t nfreqs) {
 
 void brute_fold_spectra(const float* ts_e, const float* ts_v, uint64_t nseg, uint32_t seglen,
                         const double* freqs_dev, uint32_t nfreqs, uint32_t nbins, double tsamp,
-                        double t_ref, float2* fold, void* spec, hipStream_t s) {
+                        double t_ref, float2* fold, void* spec, uint64_t spec_bytes,
+                        hipStream_t s) {
     LOKI_REQUIRE(nbins >= 2 && nbins <= 256, "Fourier brute fold: nbins must be in [2, 256]");
     LOKI_REQUIRE(seglen >= 1 && nfreqs >= 1, "Fourier brute fold: empty input");
     LOKI_REQUIRE(nseg >= 1 && 2 * nseg < (1ULL << 31), "Fourier brute fold: too many segments");
-    const auto sh = spectra_shape(seglen);
-    chunk_spectra(ts_e, ts_v, nseg, seglen, sh, spec, s);
+    const auto sh         = spectra_shape(seglen);
+    const uint64_t fit    = spec_bytes / segment_bytes(seglen);
+    LOKI_REQUIRE(fit >= 1, "Fourier brute fold: workspace below one segment's spectra");
+    const uint64_t passes = (nseg + fit - 1) / fit;
+    const uint64_t slab   = (nseg + passes - 1) / passes;
     SpecFoldArgs a{};
     a.spec   = static_cast<const float4*>(spec);
-    a.fold   = fold;
     a.freqs  = freqs_dev;
     a.nfreqs = nfreqs;
     a.nbf    = nbins / 2 + 1;
-    a.nseg   = static_cast<uint32_t>(nseg);
     a.nchunk = static_cast<uint32_t>(sh.nchunk);
     a.m      = sh.m;
     a.tsamp  = tsamp;
@@ -400,17 +412,23 @@ void brute_fold_spectra(const float* ts_e, const float* ts_v, uint64_t nseg, uin
     // where that leaves fewer than two workgroups per CU.
     constexpr uint32_t kOuts   = 4;
     constexpr uint64_t kBlocks = 512;
-    const bool wide = (lanes + kOuts * kFoldThreads - 1) / (kOuts * kFoldThreads) * nseg >= kBlocks;
+    const bool wide = (lanes + kOuts * kFoldThreads - 1) / (kOuts * kFoldThreads) * slab >= kBlocks;
     const uint32_t per = kFoldThreads * (wide ? kOuts : 1);
     a.nblk_out         = static_cast<uint32_t>((lanes + per - 1) / per);
-    // segments per workgroup: the weights (~60 operations per value) are
-    // shared by them, as long as four workgroups per CU remain
-    a.segs_per_block = static_cast<uint32_t>(
-        std::clamp<uint64_t>(nseg * a.nblk_out / (4 * kBlocks), 1, 16));
-    if (wide) {
-        launch_fold<kOuts>(a, turn, s);
-    } else {
-        launch_fold<1>(a, turn, s);
+    for (uint64_t s0 = 0; s0 < nseg; s0 += slab) {
+        const uint64_t n = std::min(slab, nseg - s0);
+        a.nseg           = static_cast<uint32_t>(n);
+        a.fold           = fold + s0 * nfreqs * 2 * a.nbf;
+        // segments per workgroup: the weights (~60 operations per value) are
+        // shared by them, as long as four workgroups per CU remain
+        a.segs_per_block =
+            static_cast<uint32_t>(std::clamp<uint64_t>(n * a.nblk_out / (4 * kBlocks), 1, 16));
+        chunk_spectra(ts_e + s0 * seglen, ts_v + s0 * seglen, n, seglen, sh, spec, s);
+        if (wide) {
+            launch_fold<kOuts>(a, turn, s);
+        } else {
+            launch_fold<1>(a, turn, s);
+        }
     }
 }
 

@@ -138,8 +138,14 @@ struct SpectraShape {
     uint64_t nchunk;
 };
 SpectraShape spectra_shape(uint64_t seglen);
-/// Bytes of the spectra of nseg segments.
-uint64_t spectra_bytes(uint64_t nseg, uint64_t seglen);
+/// Workspace of brute_fold_spectra for nseg segments: their spectra (16 bytes a
+/// sample and more), in whole segments of at most max_bytes or of one segment.
+uint64_t spectra_bytes(uint64_t nseg, uint64_t seglen, uint64_t max_bytes);
+/// max_bytes of a fold that runs in a plan's own buffers, and of one that
+/// allocates and frees it (2^23 samples: 0.3 ms for one allocation of 129 MiB, 4 ms
+/// now and then, against 0.05 ms for 64 MiB; two passes cost 0.02 to 0.08 ms).
+constexpr uint64_t kMaxSpectra       = 256ULL << 20;
+constexpr uint64_t kMaxSpectraOneOff = 64ULL << 20;
 /// Spectra of every chunk (sh.m / 2 samples) of nseg segments of both series.
 void chunk_spectra(const float* ts_e, const float* ts_v, uint64_t nseg, uint64_t seglen,
                    const SpectraShape& sh, void* spec, hipStream_t s);
@@ -147,11 +153,13 @@ void chunk_spectra(const float* ts_e, const float* ts_v, uint64_t nseg, uint64_t
 /// Whether brute_fold_spectra is the faster Fourier brute fold.
 bool spectra_fold_better(uint32_t seglen, uint32_t nfreqs);
 /// The Fourier brute fold interpolated from chunk spectra (FP64 FFTs, FP32
-/// values and weights): the same sums as brute_fold_fourier.  spec:
-/// spectra_bytes(nseg, seglen) bytes of workspace, 16-byte aligned.
+/// values and weights): the same sums as brute_fold_fourier.  spec: spec_bytes of
+/// workspace, 16-byte aligned, at least one segment's spectra; the segments
+/// are taken in as many equal passes as that needs.
 void brute_fold_spectra(const float* ts_e, const float* ts_v, uint64_t nseg, uint32_t seglen,
                         const double* freqs_dev, uint32_t nfreqs, uint32_t nbins, double tsamp,
-                        double t_ref, float2* fold, void* spec, hipStream_t s);
+                        double t_ref, float2* fold, void* spec, uint64_t spec_bytes,
+                        hipStream_t s);
 
 /// Most levels that one Fourier merge pass takes.
 constexpr uint32_t kFourierPassLevels = 3;

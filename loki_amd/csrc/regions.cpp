@@ -85,7 +85,9 @@ float FFARegionStats::cpu_memory_usage() const noexcept {
     return buffer_memory_usage() + coord_memory_usage() + extra_memory_usage();
 }
 float FFARegionStats::device_memory_usage() const noexcept {
-    // both series, the candidate scores and indices, the fold buffers and tables
+    // both series, the candidate scores and indices, the fold buffers and tables.  A
+    // Fourier chunk's spectra lie in its fold buffers; where those are smaller, at most
+    // 256 MiB beside them (kern::kMaxSpectra) come out of the planner's 0.5 GB headroom.
     const float extra = static_cast<float>((2 * m_n_samps + max_scores_size()) * sizeof(float) +
                                            max_scores_size() * sizeof(uint32_t)) /
                         kGiBf;

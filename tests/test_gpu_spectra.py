@@ -111,3 +111,55 @@ def test_series_do_not_mix():
     keep[1] = False
     assert np.array_equal(got[:, :, 1], plain[:, :, 1])
     assert np.array_equal(got[keep], plain[keep])
+
+
+def test_passes_of_segments_equal_one():
+    """A standalone fold whose spectra exceed its 64 MiB workspace runs in several passes over
+    the segments: the same bits as folding each part of the series by itself."""
+    from loki_amd import libculoki
+
+    seglen, nbins = 1000, 16
+    nseg = 3 * 4000 + 7  # 16.6 kB of spectra per segment
+    rng = np.random.default_rng(3)
+    e = rng.standard_normal(seglen * nseg, dtype=np.float32)
+    v = (0.5 + rng.random(seglen * nseg)).astype(np.float32)
+    freqs = np.linspace(10.0, 90.0, 49)
+
+    def fold(lo, hi):
+        return np.asarray(libculoki.fold.compute_brute_fold_fourier_cuda(
+            e[lo * seglen: hi * seglen], v[lo * seglen: hi * seglen], freqs, seglen, nbins, TSAMP,
+            0.0)).reshape(hi - lo, -1)
+
+    whole = fold(0, nseg)
+    for lo, hi in ((0, 2500), (2500, 6001), (6001, 9500), (9500, nseg)):
+        assert np.array_equal(whole[lo:hi], fold(lo, hi))
+
+
+@pytest.mark.parametrize(("nsamps", "lims", "bseg", "extra"), [
+    # levels larger than the spectra (65 MiB): no memory beyond the presized workspace
+    (2**22, [(20.0, 60.0)], 2048, 0),
+    # eight frequencies of long segments, levels of 0.3 MiB: the spectra (16.6 MiB) are kept
+    (2**20, [(1.0, 1.02)], 65536, 17),
+])
+def test_spectra_take_the_partner_buffer(nsamps, lims, bseg, extra):
+    import torch
+
+    from loki_amd import libculoki, libloki
+
+    cfg = libloki.configs.PulsarSearchConfig(
+        nsamps=nsamps, tsamp=TSAMP, nbins=64, eta=1.0, param_limits=np.array(lims),
+        use_fourier=True, bseg_brute=bseg)
+    e = torch.randn(nsamps, device="cuda")
+    v = torch.ones(nsamps, device="cuda")
+    plan = libculoki.ffa.FFACOMPLEXCUDA(cfg, 0).plan
+    ws = libculoki.ffa.FFAWorkspaceCUDA(device_id=0, buffer_bytes=8 * int(plan.buffer_size),
+                                        coord_bytes=16 * int(plan.coord_size))
+    ffa = libculoki.ffa.FFACOMPLEXCUDA(cfg, 0, workspace=ws)
+    fold = torch.empty(int(plan.buffer_size), dtype=torch.complex64, device="cuda")
+    torch.cuda.synchronize()
+    before = torch.cuda.mem_get_info()[0]
+    ffa.execute_device(e.data_ptr(), v.data_ptr(), fold.data_ptr(), fold.numel(), 0)
+    torch.cuda.synchronize()
+    took = (before - torch.cuda.mem_get_info()[0]) / 2**20
+    # the plan's frequencies and row terms, and the allocator's granularity: a few MiB
+    assert extra - 1 <= took <= extra + 16, took

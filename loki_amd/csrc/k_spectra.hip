@@ -372,16 +372,25 @@ void chunk_spectra(const float* ts_e, const float* ts_v, uint64_t nseg, uint64_t
     }
 }
 
-// The spectra cost the same for any number of frequencies (0.5 ms for 2^23
-// samples, workspace included), the matrix cores 2 K per value.  Measured on
-// 2^23 samples, matrix cores against spectra, nbins 16 / 64: 32 frequencies
-// 0.49 / 0.84 against 0.67 / 0.74 ms at 256 samples a segment and 0.46 / 0.73
-// against 0.52 / 0.53 ms at 2048; 256 frequencies 5.5 / 6.9 against 1.0 /
-// 2.0 ms and 3.4 / 5.3 against 0.57 / 0.77 ms.  At 8192 samples the matrix
-// cores have too few rows to fill the chip: 1.7 / 0.89 against 0.50 ms for
-// any number up to 32.
-bool spectra_fold_better(uint32_t seglen, uint32_t nfreqs) {
-    return seglen >= 64 && (nfreqs >= 48 || seglen >= 4096);
+// The spectra cost the same for any number of frequencies, the matrix cores 2 K
+// per value.  Level 0 of a plan, matrix cores against spectra, nbins 16 / 64, us:
+//   2^17 samples, segments of 64:   48 frequencies 28 / 39 against 35 / 38,
+//                                   96 frequencies 47 / 61 against 35 / 53
+//   2^17 samples, segments of 128:  48 frequencies 35 / 38 against 23 / 26
+//   2^23 samples, segments of 128:  32 frequencies 742 / 1026 (spectra about 500),
+//                                   48 frequencies 1076 / 1485 against 546 / 757
+//   2^23 samples, segments of 2048: 48 frequencies 446 / 724 against 148 / 180
+//   2^23 samples, segments of 8192: 2 frequencies 1672 / 873 against 145 / 143
+//                                   (the matrix cores have too few rows)
+// A one-off call allocates the spectra, about 25 us more: 2^17 samples, segments
+// of 128, 48 frequencies 47 / 48 against 63 / 69, 256 frequencies 85 / 129 against
+// 81 / 109; segments of 256, 64 frequencies 69 / 52 against 59 / 67.
+bool spectra_fold_better(uint64_t nseg, uint32_t seglen, uint32_t nfreqs, bool one_off) {
+    uint64_t least = seglen >= 4096 ? 1 : (seglen >= 128 ? 48 : 96);
+    if (one_off && seglen <= 256) {
+        least = std::max<uint64_t>({least, 64, (1ULL << 25) / (std::max<uint64_t>(nseg, 1) * seglen)});
+    }
+    return seglen >= 64 && nfreqs >= least;
 }
 
 void brute_fold_spectra(const float* ts_e, const float* ts_v, uint64_t nseg, uint32_t seglen,

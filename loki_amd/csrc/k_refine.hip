@@ -15,7 +15,7 @@
 // the fold is recomputed from the series for the adjoint pass.
 //
 // The sums come from chunk spectra where a candidate's phase is straight
-// enough over a chunk (spectral_ok), otherwise sample by sample:
+// enough over a chunk (takes_spectra), otherwise sample by sample:
 // phases are FP64; w_mk comes from an accurate sincospi of the FP64-reduced
 // phase and an FP32 three-term power recurrence; per-lane partial sums are
 // FP32, block and grid reductions FP64.
@@ -103,38 +103,17 @@ struct Powers {
     }
 };
 
-/// Geometry of the chunk spectra of a refinement pass (m == 0: none, every
-/// candidate goes sample by sample).
+/// Chunk spectra of a refinement pass (users.m == 0: none, every candidate goes
+/// sample by sample).
 struct RefineSpectra {
     const float4* spec;
-    uint32_t m;       ///< FFT points of a chunk of m / 2 samples
+    SpecUsers users;
     uint32_t nchunk;
-    uint32_t per;     ///< chunks per partial sum
+    uint32_t per;  ///< chunks per partial sum
 };
 
-// Over a chunk of half length D around tau_c the phase is phi_c + f_c d +
-// a_c d^2 / 2 + fddot d^3 / 6.  The spectra give the straight part exactly and
-// the quadratic one to first order; the candidate goes this way when, at the
-// highest harmonic and anywhere in the series, the quadratic part stays below
-// 2e-4 turns (its dropped square: 8e-7 rad at the ends of such a chunk) and
-// the cubic one below 1e-7 turns.  A NaN is not below.
-constexpr double kMaxQuadTurns  = 2e-4;
-constexpr double kMaxCubicTurns = 1e-7;
-
-__device__ __forceinline__ bool spectral_ok(const double* th, const RefineSpectra& sp,
-                                            uint64_t nsamps, double tsamp, double t_ref,
-                                            int top) {
-    if (sp.m == 0) {
-        return false;
-    }
-    const double d  = 0.25 * static_cast<double>(sp.m) * tsamp;
-    const double t0 = -t_ref;
-    const double t1 = (static_cast<double>(nsamps) * tsamp) - t_ref;
-    const double a  = fmax(fabs(th[1] + th[2] * t0), fabs(th[1] + th[2] * t1));
-    const double m  = static_cast<double>(top);
-    return m * a * d * d * 0.5 <= kMaxQuadTurns &&
-           m * fabs(th[2]) * d * d * d / 6.0 <= kMaxCubicTurns &&
-           fabs(th[0]) < 1e15;
+__device__ __forceinline__ bool takes_spectra(const double* th, const RefineSpectra& sp) {
+    return sp.users.m != 0 && spectral_ok(th, sp.users);
 }
 
 // Forward partials: block (chunk q, candidate c) -> part[c][q][NH][4] =
@@ -148,7 +127,7 @@ k_refine_fold(const float* __restrict__ ts_e, const float* __restrict__ ts_v, ui
               double* __restrict__ part, RefineSpectra sp) {
     __shared__ float red[kWaves][4 * NH];
     const uint32_t c  = blockIdx.y;
-    if (spectral_ok(theta + 3 * c, sp, nsamps, tsamp, t_ref, NH - 1)) {
+    if (takes_spectra(theta + 3 * c, sp)) {
         return;  // k_refine_fold_spectral's candidate
     }
     const uint64_t k0 = static_cast<uint64_t>(blockIdx.x) * chunk;
@@ -321,7 +300,7 @@ k_refine_adjoint(const float* __restrict__ ts_e, const float* __restrict__ ts_v,
     __shared__ double red[kWaves];
     __shared__ float2 s_st[2 * NH];
     const uint32_t c = blockIdx.y;
-    if (spectral_ok(theta + 3 * c, sp, nsamps, tsamp, t_ref, NH - 1)) {
+    if (takes_spectra(theta + 3 * c, sp)) {
         return;  // k_refine_adjoint_spectral's candidate
     }
     for (uint32_t i = threadIdx.x; i < 2 * NH; i += kBlock) {
@@ -409,7 +388,7 @@ __device__ __forceinline__ ChunkPhase chunk_phase(uint32_t q, uint32_t m, double
 }
 
 __device__ __forceinline__ void stage_spectrum(float4* lds, const RefineSpectra& sp, uint32_t q) {
-    const uint32_t n  = spec_stride(sp.m);
+    const uint32_t n  = spec_stride(sp.users.m);
     const float4* src = sp.spec + static_cast<uint64_t>(q) * n;
     __syncthreads();  // the previous chunk's readers are done
     for (uint32_t i = threadIdx.x; i < n; i += kBlock) {
@@ -432,7 +411,7 @@ k_refine_fold_spectral(RefineSpectra sp, uint64_t nsamps, double tsamp, double t
     const uint32_t c = blockIdx.y * kSpecCands<NH> + threadIdx.x / NH;
     const int m      = static_cast<int>(threadIdx.x % NH);
     const bool ok    = threadIdx.x < kSpecCands<NH> * NH && c < ncand &&
-                    spectral_ok(theta + 3 * c, sp, nsamps, tsamp, t_ref, NH - 1);
+                    takes_spectra(theta + 3 * c, sp);
     if (__syncthreads_or(ok) == 0) {
         return;
     }
@@ -440,7 +419,7 @@ k_refine_fold_spectral(RefineSpectra sp, uint64_t nsamps, double tsamp, double t
     const double f = th[0], fd = th[1], fdd = th[2];
     const double md    = static_cast<double>(m);
     const float quad   = -0.07957747154594767F;  // -1 / (4 pi): pi / (2 pi)^2, M in turns
-    const float mm     = static_cast<float>(sp.m);
+    const float mm     = static_cast<float>(sp.users.m);
     double er = 0.0, ei = 0.0, vr = 0.0, vi = 0.0;
     const uint32_t q0 = blockIdx.x * sp.per;
     const uint32_t q1 = min(q0 + sp.per, sp.nchunk);
@@ -450,16 +429,16 @@ k_refine_fold_spectral(RefineSpectra sp, uint64_t nsamps, double tsamp, double t
             continue;
         }
         if (m == 0) {  // the plain sums
-            const double2 dc = *reinterpret_cast<const double2*>(lds + spec_points(sp.m));
+            const double2 dc = *reinterpret_cast<const double2*>(lds + spec_points(sp.users.m));
             er += dc.x;
             vr += dc.y;
             continue;
         }
-        const ChunkPhase p = chunk_phase(q, sp.m, tsamp, t_ref, f, fd, fdd);
+        const ChunkPhase p = chunk_phase(q, sp.users.m, tsamp, t_ref, f, fd, fdd);
         const double uf    = p.fc * tsamp;
         float s, w[kSpecTaps], w1[kSpecTaps], w2[kSpecTaps];
         bool conj;
-        const uint32_t at = spec_position((uf - floor(uf)) * md, sp.m, s, conj);
+        const uint32_t at = spec_position((uf - floor(uf)) * md, sp.users.m, s, conj);
         spec_weights(s, w);
         spec_weights_d(s, w1, w2);
         // X - i pi m a tsamp^2 X2, X2 = sum x (k - C)^2 w = -(M / 2 pi)^2 X'': both real
@@ -498,14 +477,14 @@ k_refine_adjoint_spectral(RefineSpectra sp, uint64_t nsamps, double tsamp, doubl
     const uint32_t c = blockIdx.y * kSpecCands<NH> + threadIdx.x / NH;
     const int m      = static_cast<int>(threadIdx.x % NH);
     const bool ok    = threadIdx.x < kSpecCands<NH> * NH && c < ncand &&
-                    spectral_ok(theta + 3 * c, sp, nsamps, tsamp, t_ref, NH - 1);
+                    takes_spectra(theta + 3 * c, sp);
     if (__syncthreads_or(ok) == 0) {
         return;
     }
     const double* th = theta + 3 * (ok ? c : 0);
     const double f = th[0], fd = th[1], fdd = th[2];
     const double md = static_cast<double>(m);
-    const float mm  = static_cast<float>(sp.m);
+    const float mm  = static_cast<float>(sp.users.m);
     const float2 ge = state[static_cast<uint64_t>(ok ? c : 0) * (2 * NH) + m];
     const float2 gv = state[static_cast<uint64_t>(ok ? c : 0) * (2 * NH) + NH + m];
     double g0 = 0.0, g1 = 0.0, g2 = 0.0;
@@ -516,11 +495,11 @@ k_refine_adjoint_spectral(RefineSpectra sp, uint64_t nsamps, double tsamp, doubl
         if (!ok || m == 0) {
             continue;
         }
-        const ChunkPhase p = chunk_phase(q, sp.m, tsamp, t_ref, f, fd, fdd);
+        const ChunkPhase p = chunk_phase(q, sp.users.m, tsamp, t_ref, f, fd, fdd);
         const double uf    = p.fc * tsamp;
         float s, w[kSpecTaps], w1[kSpecTaps], w2[kSpecTaps];
         bool conj;
-        const uint32_t at = spec_position((uf - floor(uf)) * md, sp.m, s, conj);
+        const uint32_t at = spec_position((uf - floor(uf)) * md, sp.users.m, s, conj);
         spec_weights(s, w);
         spec_weights_d(s, w1, w2);
         const float2 z  = turns_twiddle((p.turn - floor(p.turn)) * md);
@@ -581,7 +560,10 @@ k_refine_grad_sum(const double* __restrict__ gpart, uint32_t nchunk, uint32_t nc
 
 uint32_t chunks_for(uint64_t nsamps, uint64_t ncand) {
     // about 8192 blocks in flight, chunks of >= 1024 samples; at most 256 partial
-    // sums, which one block per candidate adds up (1024 of them: 0.3 ms)
+    // sums, which one block per candidate adds up (1024 of them: 0.3 ms).  A lane of
+    // the sample loop then adds nsamps / 65536 samples or more in FP32: with 2^22
+    // samples 64, whose score is 1.3e-7 to 5.4e-7 from 64 bits for 16 to 128 bins,
+    // against 1.3e-7 to 5.4e-7 for four (the recurrence of the powers rules).
     ncand        = ncand < 1 ? 1 : ncand;
     uint64_t nq  = (8192 + ncand - 1) / ncand;
     const uint64_t max_q = std::min<uint64_t>((nsamps + 1023) / 1024, 256);
@@ -612,10 +594,11 @@ uint64_t refine_part_bytes(uint64_t nsamps, uint64_t ncand, uint32_t nbins) {
     return ncand * chunks_for(nsamps, ncand) * (4 * nh) * sizeof(double);
 }
 
-/// Spectra of the series behind the partial sums in the workspace.
-RefineSpectra refine_spectra(const float* ts_e, const float* ts_v, uint64_t nsamps,
-                             uint64_t ncand, uint32_t nbins, uint32_t nq, void* workspace,
-                             hipStream_t s) {
+/// Spectra of the series behind the partial sums in the workspace, formed if any
+/// candidate may take them.
+RefineSpectra refine_spectra(const float* ts_e, const float* ts_v, uint64_t nsamps, double tsamp,
+                             double t_ref, const double* theta, uint32_t ncand, uint32_t nbins,
+                             uint32_t nq, void* workspace, hipStream_t s) {
     RefineSpectra sp{};
     const auto sh = refine_shape(nsamps, ncand);
     if (sh.m == 0) {
@@ -624,11 +607,11 @@ RefineSpectra refine_spectra(const float* ts_e, const float* ts_v, uint64_t nsam
     LOKI_REQUIRE(sh.nchunk < (1ULL << 31), "refine: series too long");
     const auto end = reinterpret_cast<uintptr_t>(workspace) + refine_part_bytes(nsamps, ncand, nbins);
     auto* spec     = reinterpret_cast<float4*>((end + 15) & ~static_cast<uintptr_t>(15));
-    chunk_spectra(ts_e, ts_v, 1, nsamps, sh, spec, s);
     sp.spec   = spec;
-    sp.m      = sh.m;
+    sp.users  = {theta, ncand, nbins / 2, sh.m, nsamps, tsamp, t_ref};
     sp.nchunk = static_cast<uint32_t>(sh.nchunk);
     sp.per    = (sp.nchunk + nq - 1) / nq;
+    chunk_spectra(ts_e, ts_v, 1, nsamps, sh, spec, s, &sp.users);
     return sp;
 }
 
@@ -638,10 +621,11 @@ void forward_nh(const float* ts_e, const float* ts_v, uint64_t nsamps, double ts
                 uint32_t width, float* scores, float2* state, double* part, uint32_t nq,
                 hipStream_t s) {
     const uint64_t chunk = (nsamps + nq - 1) / nq;
-    const auto sp        = refine_spectra(ts_e, ts_v, nsamps, ncand, nbins, nq, part, s);
-    if (sp.m != 0) {
+    const auto sp        = refine_spectra(ts_e, ts_v, nsamps, tsamp, t_ref, theta, ncand, nbins,
+                                              nq, part, s);
+    if (sp.users.m != 0) {
         const uint32_t nc = (ncand + kSpecCands<NH> - 1) / kSpecCands<NH>;
-        k_refine_fold_spectral<NH><<<dim3(nq, nc), kBlock, spec_stride(sp.m) * sizeof(float4),
+        k_refine_fold_spectral<NH><<<dim3(nq, nc), kBlock, spec_stride(sp.users.m) * sizeof(float4),
                                      s>>>(sp, nsamps, tsamp, t_ref, theta, ncand, part);
     }
     k_refine_fold<NH><<<dim3(nq, ncand), kBlock, 0, s>>>(ts_e, ts_v, nsamps, chunk, tsamp, t_ref,
@@ -654,10 +638,11 @@ void adjoint_nh(const float* ts_e, const float* ts_v, uint64_t nsamps, double ts
                 double t_ref, const double* theta, uint32_t ncand, const float2* state,
                 double* gpart, double* grad, uint32_t nq, hipStream_t s) {
     const uint64_t chunk = (nsamps + nq - 1) / nq;
-    const auto sp = refine_spectra(ts_e, ts_v, nsamps, ncand, 2 * (NH - 1), nq, gpart, s);
-    if (sp.m != 0) {
+    const auto sp        = refine_spectra(ts_e, ts_v, nsamps, tsamp, t_ref, theta, ncand,
+                                          2 * (NH - 1), nq, gpart, s);
+    if (sp.users.m != 0) {
         const uint32_t nc = (ncand + kSpecCands<NH> - 1) / kSpecCands<NH>;
-        k_refine_adjoint_spectral<NH><<<dim3(nq, nc), kBlock, spec_stride(sp.m) * sizeof(float4),
+        k_refine_adjoint_spectral<NH><<<dim3(nq, nc), kBlock, spec_stride(sp.users.m) * sizeof(float4),
                                         s>>>(sp, nsamps, tsamp, t_ref, theta, ncand, state, gpart);
     }
     k_refine_adjoint<NH><<<dim3(nq, ncand), kBlock, 0, s>>>(ts_e, ts_v, nsamps, chunk, tsamp,

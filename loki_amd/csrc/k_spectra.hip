@@ -41,7 +41,7 @@ template <int LG> struct SpecShape {
 template <int LG>
 __global__ void __launch_bounds__(SpecShape<LG>::kThreads)
 k_chunk_spectra(const float* __restrict__ ts_e, const float* __restrict__ ts_v, uint64_t seglen,
-                uint32_t nchunk, uint64_t q0, float4* __restrict__ spec) {
+                uint32_t nchunk, uint64_t q0, float4* __restrict__ spec, SpecUsers users) {
     using S          = SpecShape<LG>;
     constexpr int M  = 1 << LG;
     constexpr int H  = S::kH;
@@ -58,6 +58,15 @@ k_chunk_spectra(const float* __restrict__ ts_e, const float* __restrict__ ts_v, 
     const uint64_t k0  = (q % nchunk) * (2 * C);
     const uint32_t len = static_cast<uint32_t>(min(static_cast<uint64_t>(2 * C), seglen - k0));
     const int tid      = static_cast<int>(threadIdx.x);
+    if (users.theta != nullptr) {  // nothing to do if no candidate reads the spectra
+        bool any = false;
+        for (uint32_t c = threadIdx.x; c < users.ncand && !any; c += T) {
+            any = spectral_ok(users.theta + 3 * static_cast<uint64_t>(c), users);
+        }
+        if (__syncthreads_or(any) == 0) {
+            return;
+        }
+    }
     const int side     = tid / TL;  // 0: e, 1: v
     const int lane     = tid % TL;
     const float* x     = (side == 0 ? ts_e : ts_v) + seg * seglen + k0;
@@ -320,11 +329,12 @@ void launch_fold(const SpecFoldArgs& a, bool turn, hipStream_t s) {
 
 template <int LG>
 void launch_spectra(const float* e, const float* v, uint64_t seglen, uint32_t nchunk, uint64_t n,
-                    float4* spec, hipStream_t s) {
+                    float4* spec, const SpecUsers& users, hipStream_t s) {
     constexpr uint64_t kMaxGrid = 1ULL << 30;
     for (uint64_t q0 = 0; q0 < n; q0 += kMaxGrid) {
         const auto g = static_cast<uint32_t>(std::min(kMaxGrid, n - q0));
-        k_chunk_spectra<LG><<<g, SpecShape<LG>::kThreads, 0, s>>>(e, v, seglen, nchunk, q0, spec);
+        k_chunk_spectra<LG><<<g, SpecShape<LG>::kThreads, 0, s>>>(e, v, seglen, nchunk, q0, spec,
+                                                          users);
     }
 }
 
@@ -357,18 +367,19 @@ uint64_t spectra_bytes(uint64_t nseg, uint64_t seglen, uint64_t max_bytes) {
 }
 
 void chunk_spectra(const float* ts_e, const float* ts_v, uint64_t nseg, uint64_t seglen,
-                   const SpectraShape& sh, void* spec, hipStream_t s) {
+                   const SpectraShape& sh, void* spec, hipStream_t s, const SpecUsers* users) {
     const uint64_t n = nseg * sh.nchunk;
     auto* out        = static_cast<float4*>(spec);
     LOKI_REQUIRE(sh.nchunk < (1ULL << 32), "chunk spectra: segment too long");
     const auto nc = static_cast<uint32_t>(sh.nchunk);
+    const SpecUsers u = users != nullptr ? *users : SpecUsers{};
     switch (sh.m) {
-    case 128: launch_spectra<7>(ts_e, ts_v, seglen, nc, n, out, s); break;
-    case 256: launch_spectra<8>(ts_e, ts_v, seglen, nc, n, out, s); break;
-    case 512: launch_spectra<9>(ts_e, ts_v, seglen, nc, n, out, s); break;
-    case 1024: launch_spectra<10>(ts_e, ts_v, seglen, nc, n, out, s); break;
-    case 2048: launch_spectra<11>(ts_e, ts_v, seglen, nc, n, out, s); break;
-    default: launch_spectra<12>(ts_e, ts_v, seglen, nc, n, out, s); break;
+    case 128: launch_spectra<7>(ts_e, ts_v, seglen, nc, n, out, u, s); break;
+    case 256: launch_spectra<8>(ts_e, ts_v, seglen, nc, n, out, u, s); break;
+    case 512: launch_spectra<9>(ts_e, ts_v, seglen, nc, n, out, u, s); break;
+    case 1024: launch_spectra<10>(ts_e, ts_v, seglen, nc, n, out, u, s); break;
+    case 2048: launch_spectra<11>(ts_e, ts_v, seglen, nc, n, out, u, s); break;
+    default: launch_spectra<12>(ts_e, ts_v, seglen, nc, n, out, u, s); break;
     }
 }
 

@@ -146,9 +146,12 @@ uint64_t spectra_bytes(uint64_t nseg, uint64_t seglen, uint64_t max_bytes);
 /// now and then, against 0.05 ms for 64 MiB; two passes cost 0.02 to 0.08 ms).
 constexpr uint64_t kMaxSpectra       = 256ULL << 20;
 constexpr uint64_t kMaxSpectraOneOff = 64ULL << 20;
+struct SpecUsers;
 /// Spectra of every chunk (sh.m / 2 samples) of nseg segments of both series.
+/// users: nothing is formed where none of these candidates may take them.
 void chunk_spectra(const float* ts_e, const float* ts_v, uint64_t nseg, uint64_t seglen,
-                   const SpectraShape& sh, void* spec, hipStream_t s);
+                   const SpectraShape& sh, void* spec, hipStream_t s,
+                   const SpecUsers* users = nullptr);
 
 /// Whether brute_fold_spectra is the faster Fourier brute fold; one_off: the
 /// workspace is allocated for the call.

@@ -125,6 +125,35 @@ __device__ __forceinline__ uint32_t spec_position(double u, uint32_t m, float& s
     return static_cast<uint32_t>(c);
 }
 
+// Over a chunk of half length D around tau_c a candidate's phase is phi_c + f_c d +
+// a_c d^2 / 2 + fddot d^3 / 6.  The spectra give the straight part exactly and
+// the quadratic one to first order; the candidate goes this way when, at the
+// highest harmonic and anywhere in the series, the quadratic part stays below
+// 2e-4 turns (its dropped square: 8e-7 rad at the ends of such a chunk) and
+// the cubic one below 1e-7 turns.  A NaN is not below.
+constexpr double kMaxQuadTurns  = 2e-4;
+constexpr double kMaxCubicTurns = 1e-7;
+
+/// Candidates (f, fdot, fddot) that may take spectra of m points over a series
+/// of nsamps; theta null: the spectra are wanted in any case.
+struct SpecUsers {
+    const double* theta;
+    uint32_t ncand, top;  ///< top: highest harmonic
+    uint32_t m;
+    uint64_t nsamps;
+    double tsamp, t_ref;
+};
+
+__device__ __forceinline__ bool spectral_ok(const double* th, const SpecUsers& u) {
+    const double d  = 0.25 * static_cast<double>(u.m) * u.tsamp;
+    const double t0 = -u.t_ref;
+    const double t1 = (static_cast<double>(u.nsamps) * u.tsamp) - u.t_ref;
+    const double a  = fmax(fabs(th[1] + th[2] * t0), fabs(th[1] + th[2] * t1));
+    const double n  = static_cast<double>(u.top);
+    return n * a * d * d * 0.5 <= kMaxQuadTurns &&
+           n * fabs(th[2]) * d * d * d / 6.0 <= kMaxCubicTurns && fabs(th[0]) < 1e15;
+}
+
 /// The chunk's (E, V) values from the 9 records at `p`.
 __device__ __forceinline__ float4 spec_value(const float4* p, const float (&w)[kSpecTaps]) {
     float4 a = make_float4(0.0F, 0.0F, 0.0F, 0.0F);

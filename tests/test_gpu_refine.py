@@ -162,6 +162,80 @@ def test_chunk_spectra_and_sample_loop_candidates(n, nbins, width):
             assert err <= 1e-5 * norm
 
 
+@pytest.mark.parametrize("n,nbins,width", [
+    (1 << 17, 16, 3),               # the shortest series and chunk with spectra
+    ((1 << 18) + 1000, 64, 2),
+    (1 << 17, 128, 5),
+])
+def test_candidates_at_the_curvature_limit(n, nbins, width):
+    """Candidates just inside and just outside the limit of the spectra: 2e-4 turns of curvature
+    at the highest harmonic, half a chunk from its centre.  Inside, each harmonic loses at most
+    8e-7 of a chunk's sum (the dropped square, at its ends), and the adjoint's first moment,
+    which has no curvature term, 2 pi 2e-4 of a term that is 1/2048 of the others (half a chunk
+    against half the series): 6e-7.  FP32 values add a few 1e-7; 1e-5 bounds the sum with a
+    margin of five.  Outside, the sample loop keeps its own bound."""
+    from loki_amd import refine
+    from oracle import refine as oref
+
+    T = n * TSAMP
+    chunk = 1 << ((n // 1024).bit_length() - 1)
+    a_max = 2 * 2e-4 / (nbins // 2 * (chunk / 2 * TSAMP) ** 2)
+    inside = [(61.7, 0.999 * a_max, 0.0), (33.1, -0.999 * a_max, 0.0),
+              (47.9, 0.0, 0.999 * a_max / (T / 2)),
+              (52.3, -0.499 * a_max, -0.5 * a_max / (T / 2))]
+    outside = [(61.7, 1.001 * a_max, 0.0), (47.9, 0.0, -1.001 * a_max / (T / 2))]
+    # pulses a tenth of a turn from the first and third: coherent sums with a gradient
+    ts_e, ts_v, t_ref = _inject(n, 83, [(61.7 + 0.1 / T, *inside[0][1:]),
+                                        (47.9 + 0.1 / T, *inside[2][1:])], [0.08, 0.08])
+    scale = np.array(refine.phase_scale(n, TSAMP, t_ref))
+    # enough harmonics in all for the spectra
+    rest = [(70.0 + k, 0.0, 0.0) for k in range(16 * 8 // (nbins // 2))]
+    th = np.array(inside + outside + rest)
+    de, dv, dth = _dev(ts_e, ts_v, th)
+    s, st = refine.score_raw(de, dv, dth, TSAMP, t_ref, nbins, width)
+    g = refine.grad_raw(de, dv, dth, st, TSAMP, t_ref, nbins).cpu().numpy()
+    s = s.cpu().numpy().astype(np.float64)
+    for c in range(len(inside) + len(outside)):
+        s_ref, g_ref = oref.grad(ts_e, ts_v, TSAMP, t_ref, th[c], nbins, width)
+        err, norm = np.linalg.norm((g[c] - g_ref) / scale), np.linalg.norm(g_ref / scale)
+        print(c, abs(s[c] - s_ref) / (1 + abs(s_ref)), err / norm)
+        if c < len(inside):
+            assert abs(s[c] - s_ref) <= 1e-5 * (1.0 + abs(s_ref))
+            assert err <= 1e-5 * norm
+        else:
+            assert abs(s[c] - s_ref) <= 1e-4 + 1e-5 * abs(s_ref)
+            assert err <= 1e-4 * norm + 2e-3
+
+
+def test_spectra_of_no_use_are_left_out():
+    """No candidate straight enough for the spectra (the FFTs are then skipped), and one in a
+    thousand that is: each as by itself."""
+    from loki_amd import refine
+
+    n, nbins, width = 1 << 17, 16, 3
+    T = n * TSAMP
+    ts_e, ts_v, t_ref = _inject(n, 91, [(61.7, 0.0, 0.0)], [0.08])
+    th = np.zeros((1000, 3))
+    th[:, 0] = np.linspace(40.0, 90.0, 1000)
+    th[:, 1] = 4.0e5 / T**2
+    de, dv = _dev(ts_e, ts_v)
+
+    def run(t):
+        (d,) = _dev(t)
+        s, st = refine.score_raw(de, dv, d, TSAMP, t_ref, nbins, width)
+        return s.cpu().numpy(), refine.grad_raw(de, dv, d, st, TSAMP, t_ref, nbins).cpu().numpy()
+
+    s, g = run(th)
+    mixed = th.copy()
+    mixed[777] = (61.7, 0.0, 0.0)
+    s2, g2 = run(mixed)
+    keep = np.arange(1000) != 777
+    assert np.array_equal(s2[keep], s[keep]) and np.array_equal(g2[keep], g[keep])
+    straight = np.tile(mixed[777], (1000, 1))
+    s3, g3 = run(straight)
+    assert s2[777] == s3[0] and np.array_equal(g2[777], g3[0])
+
+
 def _gpu_fd(de, dv, th, t_ref, nbins, width, steps):
     """Central differences of the GPU forward, one parameter at a time, for every candidate."""
     from loki_amd import refine

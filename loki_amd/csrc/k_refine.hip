@@ -573,15 +573,20 @@ uint32_t chunks_for(uint64_t nsamps, uint64_t ncand) {
 
 /// Chunks of a refinement pass: the largest power of two up to 1/1024 of the
 /// series (a candidate's drift over the series curves the phase of such a chunk
-/// by 2^-22 of it), 128 to 2048 samples.  Shorter series and few candidates go
-/// sample by sample.
-SpectraShape refine_shape(uint64_t nsamps, uint64_t ncand) {
+/// by 2^-22 of it), 128 to 2048 samples.  Shorter series go sample by sample, and
+/// so do few harmonics in all: the sample loops' time falls with candidates and
+/// harmonics, that of the FFTs and of the extra launches does not.  Forward +
+/// adjoint, sample loops against spectra, us: 2^17 samples, 9 harmonics (16 bins)
+/// 4 candidates 67 / 93, 8 75 / 92, 16 102 / 95; 17 harmonics 4 candidates
+/// 84 / 104, 8 124 / 105; 33 harmonics 4 candidates 176 / 135; 2^20 samples,
+/// 9 harmonics 8 candidates 162 / 165; 2^22 samples 4 215 / 270, 8 312 / 268.
+SpectraShape refine_shape(uint64_t nsamps, uint64_t ncand, uint32_t nbins) {
     SpectraShape sh{};
     uint32_t c = kSpecMaxC;
     while (c >= 128 && static_cast<uint64_t>(c) * 1024 > nsamps) {
         c /= 2;
     }
-    if (c < 128 || ncand < 4) {
+    if (c < 128 || ncand * (nbins / 2 + 1) < (nsamps < (1ULL << 21) ? 128 : 72)) {
         return sh;
     }
     sh.m      = 2 * c;
@@ -600,7 +605,7 @@ RefineSpectra refine_spectra(const float* ts_e, const float* ts_v, uint64_t nsam
                              double t_ref, const double* theta, uint32_t ncand, uint32_t nbins,
                              uint32_t nq, void* workspace, hipStream_t s) {
     RefineSpectra sp{};
-    const auto sh = refine_shape(nsamps, ncand);
+    const auto sh = refine_shape(nsamps, ncand, nbins);
     if (sh.m == 0) {
         return sp;
     }
@@ -653,7 +658,7 @@ void adjoint_nh(const float* ts_e, const float* ts_v, uint64_t nsamps, double ts
 }  // namespace
 
 SizeType refine_workspace_bytes(uint64_t nsamps, uint64_t ncand, uint32_t nbins) {
-    const auto sh = refine_shape(nsamps, ncand);
+    const auto sh = refine_shape(nsamps, ncand, nbins);
     return refine_part_bytes(nsamps, ncand, nbins) +
            (sh.m == 0 ? 0 : 15 + sh.nchunk * spec_stride(sh.m) * sizeof(float4));
 }

@@ -145,7 +145,10 @@ def test_chunk_spectra_and_sample_loop_candidates(n, nbins, width):
     scale = np.array(refine.phase_scale(n, TSAMP, t_ref))
     th = np.array([[61.7, 2.0 / T**2, -5.0 / T**3], [7900.1, -3.0 / T**2, 6.0 / T**3],
                    [333.3, 0.0, 0.0], [61.7, 4.0e5 / T**2, 0.0], [120.2, 1.0 / T**2, 9.0e6 / T**3]])
-    curved = np.array([False, False, False, True, True])
+    # 128 harmonics in all and more take the spectra
+    more = [[90.0 + 3.7 * k, 1.0 / T**2, 0.0] for k in range(max(0, 260 // nbins - 5))]
+    th = np.concatenate([th, np.reshape(more, (-1, 3))])
+    curved = np.isin(np.arange(th.shape[0]), [3, 4])
     de, dv, dth = _dev(ts_e, ts_v, th)
     s, st = refine.score_raw(de, dv, dth, TSAMP, t_ref, nbins, width)
     g = refine.grad_raw(de, dv, dth, st, TSAMP, t_ref, nbins).cpu().numpy()

@@ -89,7 +89,7 @@ FFABatch::FFABatch(const std::vector<SearchConfig>& cfgs, const std::vector<Size
         sr.lists = kern::build_brute_fold_lists(
             m_freqs.as<double>(), static_cast<uint32_t>(nfr),
             static_cast<uint32_t>(sr.plan.segment_lens()[0]), static_cast<uint32_t>(cfg.get_nbins()),
-            cfg.get_tsamp(), 0.0, s);
+            cfg.get_tsamp(), 0.0, kern::mean_frequency(freqs.data(), nfr), s);
     }
     build_tasks();
 }
@@ -250,7 +250,7 @@ void FFABatch::build_tasks() {
     for (uint32_t kind : {0U, 1U}) {  // 0: list path, 1: run path
         std::vector<kern::FoldTask> tasks;
         uint64_t block0 = 0;
-        uint32_t max_nbins = 0;
+        size_t lds         = 0;
         uint64_t all_segs  = 0;
         for (const auto& sr : m_series) {
             all_segs += (sr.lists.use_runs ? 1U : 0U) == kind ? sr.plan.nsegments()[0] : 0;
@@ -260,7 +260,7 @@ void FFABatch::build_tasks() {
             if ((L.use_runs ? 1U : 0U) != kind) {
                 continue;
             }
-            const uint32_t bps = kern::brute_fold_blocks_per_segment(L, all_segs);
+            const uint32_t bps = kern::brute_fold_blocks_per_segment(L, all_segs, true);
             kern::FoldTask t{};
             t.ts_e   = ts_e(static_cast<SizeType>(&sr - m_series.data()));
             t.ts_v   = ts_v(static_cast<SizeType>(&sr - m_series.data()));
@@ -279,14 +279,15 @@ void FFABatch::build_tasks() {
             t.block0 = static_cast<uint32_t>(block0);
             tasks.push_back(t);
             block0 += sr.plan.nsegments()[0] * bps;
-            max_nbins = std::max(max_nbins, L.nbins);
+            if (kind == 1) {
+                lds = std::max(lds, kern::brute_fold_runs_lds_bytes(L, bps));
+            }
         }
         LOKI_REQUIRE(block0 < (1ULL << 31), "FFABatch: brute-fold grid too large");
         if (!tasks.empty()) {
-            // fold launches keep the largest nbins of their tasks in `stride`
             m_launches.push_back({Stage::kFold, kind, static_cast<uint32_t>(tasks.size()),
                                   static_cast<uint32_t>(block0), append(blob, tasks),
-                                  max_nbins, 0, 0});
+                                  0, 0, lds});
         }
     }
     // 3. merges, one launch per level index and nbins class
@@ -468,10 +469,11 @@ void FFABatch::build_tree(std::vector<uint8_t>& blob, std::vector<SizeType>& off
         t.seglen = L.seglen;
         t.nfreqs = L.nfreqs;
         t.nbins  = L.nbins;
-        t.bps    = kern::brute_fold_blocks_per_segment(L, sr.plan.nsegments()[0]);
+        t.bps    = kern::brute_fold_blocks_per_segment(L, sr.plan.nsegments()[0], true);
         ft.push_back(t);
         const auto kind = L.use_runs ? kern::TreeKind::kFoldUnits : kern::TreeKind::kFoldList;
-        lds = std::max(lds, kern::tree_lds_bytes(kind, L.nbins, 0, 0));
+        lds = std::max(lds, L.use_runs ? kern::brute_fold_runs_lds_bytes(L, t.bps)
+                                       : kern::tree_lds_bytes(kind, 0, 0));
         fold_item[i] = add(kind, L.nbins, static_cast<uint32_t>(ft.size() - 1),
                            static_cast<uint64_t>(sr.plan.nsegments()[0]) * t.bps,
                            kern::kTreeNoDep, kern::kTreeNoDep, 0);
@@ -521,7 +523,7 @@ void FFABatch::build_tree(std::vector<uint8_t>& blob, std::vector<SizeType>& off
                                            m_sched.final_run);
                 t.unscale = 1.0F;
                 fl.push_back(t);
-                lds = std::max(lds, kern::tree_lds_bytes(kern::TreeKind::kFinal, nb, lanes,
+                lds = std::max(lds, kern::tree_lds_bytes(kern::TreeKind::kFinal, lanes,
                                                          t.fg.stride));
                 const uint32_t prev = L == 2 ? fold_item[i] : merge_item[i][L - 2];
                 add(kern::TreeKind::kFinal, nb, static_cast<uint32_t>(fl.size() - 1),
@@ -556,7 +558,7 @@ void FFABatch::enqueue(hipStream_t s) const {
             break;
         case Stage::kFold:
             kern::brute_fold_grouped(static_cast<const kern::FoldTask*>(t), ln.ntasks,
-                                     ln.nblocks, ln.nbins != 0, ln.stride, FoldStorage::kF32, s);
+                                     ln.nblocks, ln.nbins != 0, ln.lds, FoldStorage::kF32, s);
             break;
         case Stage::kMerge:
             kern::merge_grouped(static_cast<const kern::MergeTask*>(t), ln.ntasks, ln.nblocks,

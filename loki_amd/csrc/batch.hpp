@@ -96,9 +96,9 @@ private:
         uint32_t nbins;   ///< merge / final: nbins; fold: 0 list path, 1 run path
         uint32_t ntasks, nblocks;
         SizeType task_off;  ///< bytes into the task arena
-        uint32_t stride;    ///< final: LDS row stride; fold: the largest nbins
+        uint32_t stride;    ///< final: LDS row stride
         uint32_t lanes;     ///< final: lanes per trial (0: 64-lane workgroups)
-        SizeType lds;       ///< final with lanes: dynamic LDS bytes
+        SizeType lds;       ///< final with lanes, run-path fold: dynamic LDS bytes
     };
 
     int m_device;

@@ -282,7 +282,8 @@ void FFAExecutor::prepare_brute_fold(hipStream_t s) {
         // synchronises s (so `freqs` outlives the copy)
         m_bf = kern::build_brute_fold_lists(
             m_bf_freqs.as<double>(), static_cast<uint32_t>(nfreqs), static_cast<uint32_t>(seglen),
-            static_cast<uint32_t>(nbins), m_plan.config().get_tsamp(), t_ref, s);
+            static_cast<uint32_t>(nbins), m_plan.config().get_tsamp(), t_ref,
+            kern::mean_frequency(freqs.data(), nfreqs), s);
     } else {
         hip_check(hipStreamSynchronize(s), "copy brute-fold frequencies");
     }
@@ -817,7 +818,8 @@ void brute_fold_time_device(const float* ts_e, const float* ts_v, SizeType nsamp
               "copy frequencies");
     auto lists = kern::build_brute_fold_lists(
         d_freqs.as<double>(), static_cast<uint32_t>(freqs.size()),
-        static_cast<uint32_t>(segment_len), static_cast<uint32_t>(nbins), tsamp, t_ref, s);
+        static_cast<uint32_t>(segment_len), static_cast<uint32_t>(nbins), tsamp, t_ref,
+        kern::mean_frequency(freqs.data(), freqs.size()), s);
     kern::brute_fold_time(ts_e, ts_v, nsamps / segment_len, lists, fold, FoldStorage::kF32, 1.0F,
                           s);
     check_launch("brute fold launch");

@@ -185,21 +185,17 @@ __device__ __forceinline__ uint32_t run_bound(int64_t u, uint32_t n, double tsam
 // VALU and LDS are about equally busy (24 series of 2^18 to 2^21 samples,
 // 1.3e10 (sample, frequency) pairs, 3.9 ms: 9.3 lane-instructions per pair, two
 // of them the adds, and 2.8 ms of LDS cycles, 43 % of them the runs' bank
-// conflicts).  1024 pairs per block hold four blocks in a CU's LDS; 4096 pairs
-// (three blocks), every boundary by run_bound and the staging unhidden took
-// 5.3 ms.  Chunks of 4096 samples keep more lanes busy where a launch is too
-// small to fill the chip (2^20 samples, 403 frequencies, 0.5-2 Hz: 0.18
-// against 0.20 ms, 0.49 ms before; 2^17 samples 0.03 against 0.21 ms before)
-// and cost a larger one a block per CU (the batch above: 4.6 ms).
+// conflicts).  1024 pairs per block leave five blocks on a CU (26 KB of LDS, 86
+// registers); 4096 pairs (three blocks), every boundary by run_bound and the
+// staging unhidden took 5.3 ms.  Chunks of 4096 samples keep more lanes busy
+// where a launch is too small to fill the chip (2^20 samples, 403 frequencies,
+// 0.5-2 Hz: 0.18 against 0.20 ms, 0.49 ms before; 2^17 samples 0.03 against 0.21
+// ms before); they hold three blocks of 64 bins on a CU (43 KB; four by their 102
+// registers) and cost a larger launch (the batch above: 4.6 ms).
 constexpr int kUnitChunk      = 2048;  // samples staged per chunk
-constexpr int kUnitChunkSmall = 4096;  // ... in launches that leave CUs idle
+constexpr int kUnitChunkSmall = 4096;  // ... where all blocks are resident at once
 constexpr uint32_t kUnitPairs = 1024;  // (frequency, bin) pairs per block
 constexpr int kUnitMaxNF      = 64;    // frequencies per block (one wave counts their units)
-
-__host__ __device__ inline uint32_t unit_nf(uint32_t nbins) {
-    const uint32_t nf = kUnitPairs / nbins;
-    return nf < 1U ? 1U : (nf > static_cast<uint32_t>(kUnitMaxNF) ? kUnitMaxNF : nf);
-}
 
 /// What a block keeps per frequency; the chunk's part twice, in turn.
 struct UnitChunk {
@@ -213,10 +209,10 @@ struct UnitFreq {
     UnitChunk c[2];
 };
 
-__host__ __device__ inline size_t unit_lds_bytes(uint32_t nbins, int chunk = kUnitChunk) {
-    const size_t nf = unit_nf(nbins);
-    return static_cast<size_t>(chunk) * sizeof(float2) + nf * nbins * sizeof(float2) + nf * sizeof(UnitFreq) +
-           2 * sizeof(uint32_t);
+/// LDS of a block of nf frequencies.
+inline size_t unit_lds_bytes(uint32_t nf, uint32_t nbins, int chunk) {
+    return static_cast<size_t>(chunk) * sizeof(float2) +
+           nf * (nbins * sizeof(float2) + sizeof(UnitFreq)) + 2 * sizeof(uint32_t);
 }
 
 /// First sample of the chunk at or after the beginning of bin ulo + i: the
@@ -246,7 +242,7 @@ __device__ __forceinline__ void bf_units_block(uint32_t bid, const float* __rest
                                                double t_ref, TO* __restrict__ fold, float scale) {
     constexpr int kPre = CHUNK / kFoldBlock;  // samples a lane stages per chunk
     extern __shared__ __align__(16) unsigned char s_mem[];
-    const uint32_t NF  = (nfreqs + blocks_per_seg - 1) / blocks_per_seg;  // <= unit_nf(nbins)
+    const uint32_t NF  = (nfreqs + blocks_per_seg - 1) / blocks_per_seg;
     auto* s_ev         = reinterpret_cast<float2*>(s_mem);  // [CHUNK], 16-byte aligned
     auto* acc          = s_ev + CHUNK;                   // [NF][nbins]
     auto* fq           = reinterpret_cast<UnitFreq*>(acc + NF * nbins);  // [NF]

@@ -12,6 +12,7 @@
 // sum once (storage.hpp).
 #include <algorithm>
 #include <array>
+#include <cmath>
 #include <mutex>
 #include <type_traits>
 #include <vector>
@@ -274,7 +275,7 @@ k_bf_units_grouped(const FoldTask* __restrict__ tasks, uint32_t ntasks) {
 }  // namespace
 
 BruteFoldLists build_brute_fold_lists(const double* freqs_dev, uint32_t nfreqs, uint32_t seglen,
-                                      uint32_t nbins, double tsamp, double t_ref,
+                                      uint32_t nbins, double tsamp, double t_ref, double f_mean,
                                       hipStream_t s) {
     LOKI_REQUIRE(nbins >= 1 && nbins <= 1024, "brute fold supports 1 <= nbins <= 1024");
     LOKI_REQUIRE(nfreqs >= 1 && seglen >= 1, "brute fold: empty frequency or segment");
@@ -285,6 +286,7 @@ BruteFoldLists build_brute_fold_lists(const double* freqs_dev, uint32_t nfreqs, 
     L.nbins    = nbins;
     L.tsamp    = tsamp;
     L.t_ref    = t_ref;
+    L.f_mean   = f_mean;
     L.use_runs = seglen > static_cast<uint32_t>(kLdsSamps);
     L.freqs.reserve(static_cast<SizeType>(nfreqs) * sizeof(double));
     hip_check(hipMemcpyAsync(L.freqs.get(), freqs_dev, nfreqs * sizeof(double),
@@ -357,7 +359,52 @@ unsigned char* scratch_address() {
 
 constexpr uint64_t align256(uint64_t x) { return (x + 255) & ~static_cast<uint64_t>(255); }
 
-constexpr uint64_t kUnitBlocks = 512;  // two per CU
+constexpr uint64_t kCus              = 256;
+constexpr uint64_t kSmallChunkBlocks = 4;  // per CU, by registers
+constexpr uint64_t kLdsPerCu         = 160 * 1024;
+
+/// Blocks of nf frequencies with chunks of 4096 samples the chip holds at once.
+uint64_t resident_small(uint32_t nf, uint32_t nbins) {
+    return kCus * std::min<uint64_t>(kSmallChunkBlocks,
+                                     kLdsPerCu / unit_lds_bytes(nf, nbins, kUnitChunkSmall));
+}
+
+/// Frequencies per block of the run path: 1024 (frequency, bin) pairs, up to
+/// 2048 in a large launch whose chunks of 2048 samples hold fewer than a unit per
+/// lane (not in a grouped launch, where the larger blocks' LDS takes one block
+/// per CU from every series: the batch of 24 series 5.95 against 5.52 ms); fewer
+/// frequencies, down to 8, where that leaves less than two blocks per CU.
+/// Standalone folds of 0.3-1 Hz, 1024 against 2048 pairs: 2^22 samples in segments
+/// of 4608, 40 frequencies, 1000 bins (about 86 units) 0.34 against 0.28 ms, 400
+/// frequencies, 512 bins (44 units) 1.56 against 1.31 ms; of 3-12 Hz (500 units)
+/// 2048 pairs take 1.2 times as long; in segments of 131072, 40 frequencies, 512
+/// bins (640 blocks) 0.20 against 0.26 ms.  Under 8: 2^20 samples, 403 frequencies,
+/// 64 bins 0.29 ms at 4 against 0.20.  2^22 samples in segments of 131072, 400
+/// frequencies, 64 bins, 16 per block: 800 blocks 0.60 ms, 17: 768, all resident, 0.47.
+uint32_t unit_nf(const BruteFoldView& L, uint64_t nseg, bool grouped) {
+    uint32_t nf    = std::clamp<uint32_t>(kUnitPairs / L.nbins, 1, kUnitMaxNF);
+    auto blocks    = [&](uint32_t n) { return nseg * ((L.nfreqs + n - 1) / n); };
+    const double b = 1.0 + std::fabs(L.f_mean) * L.tsamp * kUnitChunk * L.nbins;
+    const double u = b < L.nbins ? b : L.nbins;
+    if (!grouped && nf * u < kFoldBlock && 2 * nf <= kUnitMaxNF &&
+        2 * nf * L.nbins <= 2 * kUnitPairs && blocks(2 * nf) >= 4 * kCus) {
+        return 2 * nf;
+    }
+    while (nf > 8 && blocks(nf) < 2 * kCus) {
+        nf = (nf + 1) / 2;
+    }
+    // up to a quarter more frequencies where that makes all blocks resident
+    const uint64_t fit = resident_small(nf, L.nbins);
+    if (!grouped && blocks(nf) > fit && nseg <= fit) {
+        const auto per    = static_cast<uint32_t>(fit / nseg);
+        const uint32_t n2 = (L.nfreqs + per - 1) / per;
+        if (4 * n2 <= 5 * nf && n2 <= static_cast<uint32_t>(kUnitMaxNF) &&
+            blocks(n2) <= resident_small(n2, L.nbins)) {
+            return n2;
+        }
+    }
+    return nf;
+}
 
 /// Segments per block of the list fold: as many as fit 32 KB of LDS (8 B per
 /// sample), at most 8; 1 selects the one-segment kernel.
@@ -376,13 +423,18 @@ void launch_fold(const float* ts_e, const float* ts_v, uint64_t blocks, uint32_t
     if (L.use_runs) {
         const auto g = static_cast<unsigned>(blocks);
         const auto* fr = L.freqs;
-        if (blocks < 2 * kUnitBlocks) {
+        // Large chunks only where every block is resident at once: a second round
+        // of blocks costs more than they give (2^22 samples in 128 segments, 400
+        // frequencies of 0.3-1 Hz, 8 bins, 896 blocks of three a CU: 0.54 against
+        // 0.40 ms in chunks of 2048).
+        const uint32_t nf = (L.nfreqs + bps - 1) / bps;
+        if (blocks <= resident_small(nf, L.nbins)) {
             k_bf_units<TO, kUnitChunkSmall>
-                <<<g, kBlock, unit_lds_bytes(L.nbins, kUnitChunkSmall), s>>>(
+                <<<g, kBlock, unit_lds_bytes(nf, L.nbins, kUnitChunkSmall), s>>>(
                     ts_e, ts_v, L.seglen, L.nfreqs, L.nbins, bps, fr, L.tsamp, L.t_ref, fold,
                     scale);
         } else {
-            k_bf_units<TO, kUnitChunk><<<g, kBlock, unit_lds_bytes(L.nbins), s>>>(
+            k_bf_units<TO, kUnitChunk><<<g, kBlock, unit_lds_bytes(nf, L.nbins, kUnitChunk), s>>>(
                 ts_e, ts_v, L.seglen, L.nfreqs, L.nbins, bps, fr, L.tsamp, L.t_ref, fold, scale);
         }
     } else if (fold_segs_per_block(L.seglen) > 1) {
@@ -422,7 +474,7 @@ void brute_fold_time(const float* ts_e, const float* ts_v, uint64_t nseg,
 void brute_fold_time(const float* ts_e, const float* ts_v, uint64_t nseg,
                      const BruteFoldView& L, void* fold, FoldStorage so, float scale,
                      hipStream_t s) {
-    const uint32_t bps    = brute_fold_blocks_per_segment(L, nseg);
+    const uint32_t bps    = brute_fold_blocks_per_segment(L, nseg, false);
     const uint64_t blocks = nseg * bps;
     LOKI_REQUIRE(blocks < (1ULL << 31), "brute fold grid too large");
     if (blocks == 0) {
@@ -468,6 +520,7 @@ void brute_fold_time_noalloc(const float* ts_e, const float* ts_v, uint64_t nsam
     v.nbins    = nbins;
     v.tsamp    = tsamp;
     v.t_ref    = t_ref;
+    v.f_mean   = mean_frequency(freqs_host, nfreqs);
     v.use_runs = seglen > static_cast<uint32_t>(kLdsSamps);
     const uint64_t need = v.use_runs ? static_cast<uint64_t>(nfreqs) * sizeof(double) : o_list;
     if (need > kScratchBytes) {
@@ -518,19 +571,13 @@ void brute_fold_time_noalloc(const float* ts_e, const float* ts_v, uint64_t nsam
     hip_check(hipStreamSynchronize(s), "brute fold");
 }
 
-uint32_t brute_fold_blocks_per_segment(const BruteFoldLists& L, uint64_t nseg) {
-    return brute_fold_blocks_per_segment(L.view(), nseg);
+uint32_t brute_fold_blocks_per_segment(const BruteFoldLists& L, uint64_t nseg, bool grouped) {
+    return brute_fold_blocks_per_segment(L.view(), nseg, grouped);
 }
 
-uint32_t brute_fold_blocks_per_segment(const BruteFoldView& L, uint64_t nseg) {
+uint32_t brute_fold_blocks_per_segment(const BruteFoldView& L, uint64_t nseg, bool grouped) {
     if (L.use_runs) {
-        // Few segments: fewer frequencies per block, down to 8 (fewer leave too
-        // few units per chunk: 0.29 against 0.20 ms at 4 with 2^20 samples, 403
-        // frequencies, 64 bins), until there are two blocks per CU.
-        uint32_t nf = unit_nf(L.nbins);
-        while (nf > 8 && nseg * ((L.nfreqs + nf - 1) / nf) < kUnitBlocks) {
-            nf = (nf + 1) / 2;
-        }
+        const uint32_t nf = unit_nf(L, nseg, grouped);
         return (L.nfreqs + nf - 1) / nf;
     }
     const uint64_t pairs = static_cast<uint64_t>(L.nfreqs) * L.nbins;
@@ -538,22 +585,30 @@ uint32_t brute_fold_blocks_per_segment(const BruteFoldView& L, uint64_t nseg) {
     return static_cast<uint32_t>((pairs + kPairsBlk - 1) / kPairsBlk);
 }
 
+size_t brute_fold_runs_lds_bytes(const BruteFoldLists& L, uint32_t bps) {
+    return unit_lds_bytes((L.nfreqs + bps - 1) / bps, L.nbins, kUnitChunk);
+}
+
+double mean_frequency(const double* freqs, uint64_t n) {
+    double sum = 0.0;
+    for (uint64_t i = 0; i < n; ++i) {
+        sum += freqs[i];
+    }
+    return n > 0 ? sum / static_cast<double>(n) : 0.0;
+}
+
 template <typename TO>
 void grouped_fold(const FoldTask* tasks, uint32_t ntasks, uint32_t nblocks, bool runs,
-                  uint32_t max_nbins, hipStream_t s) {
+                  size_t lds, hipStream_t s) {
     if (!runs) {
         k_bf_fold_grouped<true, TO><<<nblocks, kBlock, 0, s>>>(tasks, ntasks);
         return;
-    }
-    size_t lds = 0;  // enough for every nbins up to the launch's largest
-    for (uint32_t nb = 1; nb <= max_nbins; ++nb) {
-        lds = std::max(lds, unit_lds_bytes(nb));
     }
     k_bf_units_grouped<TO><<<nblocks, kBlock, lds, s>>>(tasks, ntasks);
 }
 
 void brute_fold_grouped(const FoldTask* tasks, uint32_t ntasks, uint32_t nblocks, bool runs,
-                        uint32_t max_nbins, FoldStorage so, hipStream_t s) {
+                        size_t lds, FoldStorage so, hipStream_t s) {
     if (ntasks == 0 || nblocks == 0) {
         return;
     }
@@ -562,11 +617,11 @@ void brute_fold_grouped(const FoldTask* tasks, uint32_t ntasks, uint32_t nblocks
         LOKI_REQUIRE(false, "grouped brute fold: block floating point unsupported");
         return;
     case FoldStorage::kF32:
-        return grouped_fold<float>(tasks, ntasks, nblocks, runs, max_nbins, s);
+        return grouped_fold<float>(tasks, ntasks, nblocks, runs, lds, s);
     case FoldStorage::kF16:
-        return grouped_fold<_Float16>(tasks, ntasks, nblocks, runs, max_nbins, s);
+        return grouped_fold<_Float16>(tasks, ntasks, nblocks, runs, lds, s);
     case FoldStorage::kBF16:
-        return grouped_fold<__bf16>(tasks, ntasks, nblocks, runs, max_nbins, s);
+        return grouped_fold<__bf16>(tasks, ntasks, nblocks, runs, lds, s);
     }
 }
 

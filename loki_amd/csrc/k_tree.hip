@@ -213,10 +213,9 @@ k_tree(TreeArgs a) {
 
 }  // namespace
 
-size_t tree_lds_bytes(TreeKind kind, uint32_t nbins, uint32_t lanes, uint32_t stride) {
+size_t tree_lds_bytes(TreeKind kind, uint32_t lanes, uint32_t stride) {
     switch (kind) {
     case TreeKind::kFoldList: return 2 * static_cast<size_t>(kLdsSamps) * sizeof(float);
-    case TreeKind::kFoldUnits: return unit_lds_bytes(nbins);
     case TreeKind::kFinal: return final_wide_lds_bytes(lanes, stride);
     default: return 0;
     }

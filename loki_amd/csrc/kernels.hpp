@@ -63,6 +63,7 @@ struct BruteFoldView {
     bool use_runs{false};
     double tsamp{0.0};
     double t_ref{0.0};
+    double f_mean{0.0};              ///< sizes the run path's blocks
     const double* freqs{nullptr};    ///< f64 [nfreqs]
     const uint32_t* counts{nullptr};  ///< u32 [nfreqs * nbins]
     const uint64_t* base{nullptr};    ///< u64 [nfreqs]
@@ -75,19 +76,24 @@ struct BruteFoldLists {
     bool use_runs{false};
     double tsamp{0.0};
     double t_ref{0.0};
+    double f_mean{0.0};
     DeviceBuffer freqs;   ///< f64 [nfreqs]
     DeviceBuffer counts;  ///< u32 [nfreqs * nbins]
     DeviceBuffer base;    ///< u64 [nfreqs]
     DeviceBuffer list;    ///< u32 [sum_f kmax_f * nbins]
     BruteFoldView view() const {
-        return {nfreqs, seglen, nbins, use_runs, tsamp, t_ref,
+        return {nfreqs, seglen, nbins, use_runs, tsamp, t_ref, f_mean,
                 freqs.as<double>(), counts.as<uint32_t>(), base.as<uint64_t>(),
                 list.as<uint32_t>()};
     }
 };
-/// FP64 phase bins (psr_utils.hpp:53-63) -> lists; synchronises `s`.
+/// Mean of n host frequencies.
+double mean_frequency(const double* freqs, uint64_t n);
+/// FP64 phase bins (psr_utils.hpp:53-63) -> lists; synchronises `s`.  f_mean: the
+/// frequencies' mean (it decides how the run path is split, not its result).
 BruteFoldLists build_brute_fold_lists(const double* freqs_dev, uint32_t nfreqs, uint32_t seglen,
-                                      uint32_t nbins, double tsamp, double t_ref, hipStream_t s);
+                                      uint32_t nbins, double tsamp, double t_ref, double f_mean,
+                                      hipStream_t s);
 /// fold[nseg, nfreqs, 2, nbins] = ascending-order bucket sums of each segment
 /// (FP32), stored as `so`; unless so is FP32 each sum is multiplied by
 /// `scale` before rounding.
@@ -355,15 +361,17 @@ void resolve_grouped(const ResolveTask* tasks, uint32_t ntasks, uint32_t nblocks
                      hipStream_t s);
 /// Blocks per segment of the time brute fold of `lists` (list or run path;
 /// tasks of one grouped launch must share the path).
-/// nseg: segments the launch folds (all its tasks' together): few take more
-/// blocks each.
-uint32_t brute_fold_blocks_per_segment(const BruteFoldLists& lists, uint64_t nseg);
-uint32_t brute_fold_blocks_per_segment(const BruteFoldView& lists, uint64_t nseg);
+/// nseg: segments the launch folds (all its tasks' together); grouped: other
+/// series are in it.
+uint32_t brute_fold_blocks_per_segment(const BruteFoldLists& lists, uint64_t nseg, bool grouped);
+uint32_t brute_fold_blocks_per_segment(const BruteFoldView& lists, uint64_t nseg, bool grouped);
+/// Dynamic LDS of a run-path block where `bps` blocks take a segment.
+size_t brute_fold_runs_lds_bytes(const BruteFoldLists& lists, uint32_t bps);
 /// Grouped time brute fold (all tasks stored as `so`): the list path, or with
-/// `runs` the long-segment run path (max_nbins: the largest nbins of the
-/// tasks, which sizes its LDS).
+/// `runs` the long-segment run path (lds: the largest
+/// brute_fold_runs_lds_bytes of the tasks).
 void brute_fold_grouped(const FoldTask* tasks, uint32_t ntasks, uint32_t nblocks, bool runs,
-                        uint32_t max_nbins, FoldStorage so, hipStream_t s);
+                        size_t lds, FoldStorage so, hipStream_t s);
 /// Grouped merges of one storage type, nbins and coordinate kind.
 void merge_grouped(const MergeTask* tasks, uint32_t ntasks, uint32_t nblocks, uint32_t nbins,
                    bool poly, FoldStorage st, hipStream_t s);
@@ -443,9 +451,9 @@ struct TreeArgs {
     uint32_t* sync;
     uint32_t spin_limit;
 };
-/// Dynamic LDS bytes of one item kind (fold: its nbins; final: nbins, lanes
-/// and the LDS row stride of final_lds_stride).
-size_t tree_lds_bytes(TreeKind kind, uint32_t nbins, uint32_t lanes, uint32_t stride);
+/// Dynamic LDS bytes of one item kind (final: lanes and the LDS row stride of
+/// final_lds_stride), brute_fold_runs_lds_bytes for kFoldUnits.
+size_t tree_lds_bytes(TreeKind kind, uint32_t lanes, uint32_t stride);
 /// Workgroups of 256 lanes resident at once with `lds` bytes each.
 uint32_t tree_resident_blocks(size_t lds);
 /// One persistent launch of nblocks workgroups over every ticket.

@@ -1103,6 +1103,7 @@ PYBIND11_MODULE(_loki_amd, m) {
              py::arg("find_max") = false)
         .def("set_timing", &FFA::set_timing, py::arg("enable"))
         .def("set_fused", &FFA::set_fused, py::arg("enable"))
+        .def("set_two_level_merges", &FFA::set_two_level_merges, py::arg("enable"))
         .def("set_exact_norm", &FFA::set_exact_norm, py::arg("exact"))
         .def("set_dft_precision", &FFA::set_dft_precision, py::arg("precision"))
         .def("scores_filter", &FFA::scores_filter_host, py::arg("ts_e"), py::arg("ts_v"),

@@ -31,6 +31,14 @@ CASES = {
     # 2x1, 3x4, 2x4
     "freq_50_deep": (2**18, 50, [(5.0, 230.0)], 2048),
 }
+# the level each pass ends at, as the timing records give it
+PASS_ENDS = {
+    "accel_64": [1, 4, 6],
+    "accel_50_grows": [1, 3, 5, 6, 7],
+    "freq_64": [1, 4, 6],
+    "freq_50": [1, 3, 5],
+    "freq_50_deep": [2, 5, 7],
+}
 
 
 @pytest.mark.parametrize("name", list(CASES))
@@ -45,8 +53,18 @@ def test_fourier_passes_within_bound(oracle, name):
     ocfg = SearchConfig(nsamps, TSAMP, nbins, 1.0, lims, use_fourier=True, bseg_brute=bseg)
     ts_e, ts_v = _series(nsamps, seed=31)
     ffa = libculoki.ffa.FFACOMPLEXCUDA(cfg, device_id=0)
+    ffa.set_timing(True)
     got = np.zeros(ffa.plan.buffer_size, dtype=np.complex64)
     ffa.execute(ts_e, ts_v, got)
+    assert [level for kind, level, _ in ffa.timings() if kind == "merge"] == PASS_ENDS[name]
+    # one pass per level: the same bits
+    ffa.set_two_level_merges(False)
+    single = np.zeros_like(got)
+    ffa.execute(ts_e, ts_v, single)
+    assert [level for kind, level, _ in ffa.timings() if kind == "merge"] == \
+        list(range(1, int(ffa.plan.n_levels)))
+    size = int(ffa.plan.fold_size)
+    np.testing.assert_array_equal(got[:size].view(np.float32), single[:size].view(np.float32))
     want, _ = oracle.compute_ffa(ts_e, ts_v, ocfg, fourier=True)
     _row_check(got[: ffa.plan.fold_size], want, nbins // 2 + 1, 1e-5, name)
 

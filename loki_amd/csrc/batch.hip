@@ -252,15 +252,23 @@ void FFABatch::build_tasks() {
         uint64_t block0 = 0;
         size_t lds         = 0;
         uint64_t all_segs  = 0;
+        double work = 0.0, few = 0.0;  // (sample, frequency) pairs, those of few-unit series
         for (const auto& sr : m_series) {
-            all_segs += (sr.lists.use_runs ? 1U : 0U) == kind ? sr.plan.nsegments()[0] : 0;
+            const auto& L = sr.lists;
+            if ((L.use_runs ? 1U : 0U) == kind) {
+                const double w = static_cast<double>(sr.plan.config().get_nsamps()) * L.nfreqs;
+                all_segs += sr.plan.nsegments()[0];
+                work += w;
+                few += kern::brute_fold_few_units(L.view()) ? w : 0.0;
+            }
         }
+        const auto rb = 2.0 * few > work ? kern::RunBlocks::kGroupedWide : kern::RunBlocks::kGrouped;
         for (const auto& sr : m_series) {
             const auto& L = sr.lists;
             if ((L.use_runs ? 1U : 0U) != kind) {
                 continue;
             }
-            const uint32_t bps = kern::brute_fold_blocks_per_segment(L, all_segs, true);
+            const uint32_t bps = kern::brute_fold_blocks_per_segment(L, all_segs, rb);
             kern::FoldTask t{};
             t.ts_e   = ts_e(static_cast<SizeType>(&sr - m_series.data()));
             t.ts_v   = ts_v(static_cast<SizeType>(&sr - m_series.data()));
@@ -469,7 +477,8 @@ void FFABatch::build_tree(std::vector<uint8_t>& blob, std::vector<SizeType>& off
         t.seglen = L.seglen;
         t.nfreqs = L.nfreqs;
         t.nbins  = L.nbins;
-        t.bps    = kern::brute_fold_blocks_per_segment(L, sr.plan.nsegments()[0], true);
+        t.bps    = kern::brute_fold_blocks_per_segment(L, sr.plan.nsegments()[0],
+                                                       kern::RunBlocks::kGrouped);
         ft.push_back(t);
         const auto kind = L.use_runs ? kern::TreeKind::kFoldUnits : kern::TreeKind::kFoldList;
         lds = std::max(lds, L.use_runs ? kern::brute_fold_runs_lds_bytes(L, t.bps)

@@ -369,11 +369,14 @@ uint64_t resident_small(uint32_t nf, uint32_t nbins) {
                                      kLdsPerCu / unit_lds_bytes(nf, nbins, kUnitChunkSmall));
 }
 
-/// Frequencies per block of the run path: 1024 (frequency, bin) pairs, up to
-/// 2048 in a large launch whose chunks of 2048 samples hold fewer than a unit per
-/// lane (not in a grouped launch, where the larger blocks' LDS takes one block
-/// per CU from every series: the batch of 24 series 5.95 against 5.52 ms); fewer
-/// frequencies, down to 8, where that leaves less than two blocks per CU.
+uint32_t frequencies_of(uint32_t pairs, uint32_t nbins) {
+    return std::clamp<uint32_t>(pairs / nbins, 1, kUnitMaxNF);
+}
+
+/// Frequencies per block of the run path: 1024 (frequency, bin) pairs, 2048 in a
+/// large launch whose chunks of 2048 samples hold fewer than a unit per lane
+/// (brute_fold_few_units); fewer frequencies, down to 8, where that leaves less
+/// than two blocks per CU.
 /// Standalone folds of 0.3-1 Hz, 1024 against 2048 pairs: 2^22 samples in segments
 /// of 4608, 40 frequencies, 1000 bins (about 86 units) 0.34 against 0.28 ms, 400
 /// frequencies, 512 bins (44 units) 1.56 against 1.31 ms; of 3-12 Hz (500 units)
@@ -381,21 +384,27 @@ uint64_t resident_small(uint32_t nf, uint32_t nbins) {
 /// bins (640 blocks) 0.20 against 0.26 ms.  Under 8: 2^20 samples, 403 frequencies,
 /// 64 bins 0.29 ms at 4 against 0.20.  2^22 samples in segments of 131072, 400
 /// frequencies, 64 bins, 16 per block: 800 blocks 0.60 ms, 17: 768, all resident, 0.47.
-uint32_t unit_nf(const BruteFoldView& L, uint64_t nseg, bool grouped) {
-    uint32_t nf    = std::clamp<uint32_t>(kUnitPairs / L.nbins, 1, kUnitMaxNF);
-    auto blocks    = [&](uint32_t n) { return nseg * ((L.nfreqs + n - 1) / n); };
-    const double b = 1.0 + std::fabs(L.f_mean) * L.tsamp * kUnitChunk * L.nbins;
-    const double u = b < L.nbins ? b : L.nbins;
-    if (!grouped && nf * u < kFoldBlock && 2 * nf <= kUnitMaxNF &&
-        2 * nf * L.nbins <= 2 * kUnitPairs && blocks(2 * nf) >= 4 * kCus) {
-        return 2 * nf;
+/// Grouped launches take one size for all their series (the largest block's LDS
+/// is every block's: the batch of 24 series 5.95 ms with sizes mixed, 5.52 with
+/// 1024): batches of 0.2-6 Hz, where series of few units have 84 to 100 % of the
+/// work, 256 series 71.3 against 62.8 ms, 64 series 14.5 against 12.8, 8 series
+/// 1.80 against 1.72; batches of 0.5-20 Hz (0 to 23 %), 20 series 4.73 against
+/// 5.23 ms, 7 series 0.55 against 0.67.
+uint32_t unit_nf(const BruteFoldView& L, uint64_t nseg, RunBlocks rb) {
+    uint32_t nf = frequencies_of(rb == RunBlocks::kGroupedWide ? 2 * kUnitPairs : kUnitPairs, L.nbins);
+    auto blocks = [&](uint32_t n) { return nseg * ((L.nfreqs + n - 1) / n); };
+    if (rb == RunBlocks::kAlone && brute_fold_few_units(L)) {
+        const uint32_t wide = frequencies_of(2 * kUnitPairs, L.nbins);
+        if (blocks(wide) >= 4 * kCus) {
+            return wide;
+        }
     }
     while (nf > 8 && blocks(nf) < 2 * kCus) {
         nf = (nf + 1) / 2;
     }
     // up to a quarter more frequencies where that makes all blocks resident
     const uint64_t fit = resident_small(nf, L.nbins);
-    if (!grouped && blocks(nf) > fit && nseg <= fit) {
+    if (rb == RunBlocks::kAlone && blocks(nf) > fit && nseg <= fit) {
         const auto per    = static_cast<uint32_t>(fit / nseg);
         const uint32_t n2 = (L.nfreqs + per - 1) / per;
         if (4 * n2 <= 5 * nf && n2 <= static_cast<uint32_t>(kUnitMaxNF) &&
@@ -474,7 +483,7 @@ void brute_fold_time(const float* ts_e, const float* ts_v, uint64_t nseg,
 void brute_fold_time(const float* ts_e, const float* ts_v, uint64_t nseg,
                      const BruteFoldView& L, void* fold, FoldStorage so, float scale,
                      hipStream_t s) {
-    const uint32_t bps    = brute_fold_blocks_per_segment(L, nseg, false);
+    const uint32_t bps    = brute_fold_blocks_per_segment(L, nseg, RunBlocks::kAlone);
     const uint64_t blocks = nseg * bps;
     LOKI_REQUIRE(blocks < (1ULL << 31), "brute fold grid too large");
     if (blocks == 0) {
@@ -571,18 +580,24 @@ void brute_fold_time_noalloc(const float* ts_e, const float* ts_v, uint64_t nsam
     hip_check(hipStreamSynchronize(s), "brute fold");
 }
 
-uint32_t brute_fold_blocks_per_segment(const BruteFoldLists& L, uint64_t nseg, bool grouped) {
-    return brute_fold_blocks_per_segment(L.view(), nseg, grouped);
+uint32_t brute_fold_blocks_per_segment(const BruteFoldLists& L, uint64_t nseg, RunBlocks rb) {
+    return brute_fold_blocks_per_segment(L.view(), nseg, rb);
 }
 
-uint32_t brute_fold_blocks_per_segment(const BruteFoldView& L, uint64_t nseg, bool grouped) {
+uint32_t brute_fold_blocks_per_segment(const BruteFoldView& L, uint64_t nseg, RunBlocks rb) {
     if (L.use_runs) {
-        const uint32_t nf = unit_nf(L, nseg, grouped);
+        const uint32_t nf = unit_nf(L, nseg, rb);
         return (L.nfreqs + nf - 1) / nf;
     }
     const uint64_t pairs = static_cast<uint64_t>(L.nfreqs) * L.nbins;
     LOKI_REQUIRE(pairs < (1ULL << 31), "brute fold: too many (freq, bin) pairs");
     return static_cast<uint32_t>((pairs + kPairsBlk - 1) / kPairsBlk);
+}
+
+bool brute_fold_few_units(const BruteFoldView& L) {
+    const double b = 1.0 + std::fabs(L.f_mean) * L.tsamp * kUnitChunk * L.nbins;
+    const double u = b < L.nbins ? b : L.nbins;
+    return std::clamp<uint32_t>(kUnitPairs / L.nbins, 1, kUnitMaxNF) * u < kFoldBlock;
 }
 
 size_t brute_fold_runs_lds_bytes(const BruteFoldLists& L, uint32_t bps) {

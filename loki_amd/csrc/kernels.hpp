@@ -359,12 +359,16 @@ struct FinalTask {
 /// Grouped FP64 shift tables (np == 1 or poly, one kind per launch).
 void resolve_grouped(const ResolveTask* tasks, uint32_t ntasks, uint32_t nblocks, uint32_t np,
                      hipStream_t s);
+/// Run-path blocks of a launch: one fold's, or (grouped) one size for many series.
+enum class RunBlocks { kAlone, kGrouped, kGroupedWide };
 /// Blocks per segment of the time brute fold of `lists` (list or run path;
 /// tasks of one grouped launch must share the path).
-/// nseg: segments the launch folds (all its tasks' together); grouped: other
-/// series are in it.
-uint32_t brute_fold_blocks_per_segment(const BruteFoldLists& lists, uint64_t nseg, bool grouped);
-uint32_t brute_fold_blocks_per_segment(const BruteFoldView& lists, uint64_t nseg, bool grouped);
+/// nseg: segments the launch folds (all its tasks' together).
+uint32_t brute_fold_blocks_per_segment(const BruteFoldLists& lists, uint64_t nseg, RunBlocks rb);
+uint32_t brute_fold_blocks_per_segment(const BruteFoldView& lists, uint64_t nseg, RunBlocks rb);
+/// Whether a chunk of the run path holds fewer units than a block has lanes, for
+/// the block's frequencies: such folds take wide blocks in a large launch.
+bool brute_fold_few_units(const BruteFoldView& lists);
 /// Dynamic LDS of a run-path block where `bps` blocks take a segment.
 size_t brute_fold_runs_lds_bytes(const BruteFoldLists& lists, uint32_t bps);
 /// Grouped time brute fold (all tasks stored as `so`): the list path, or with

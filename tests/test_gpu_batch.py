@@ -60,6 +60,28 @@ def test_batch_matches_oracle_and_single_series(oracle):
     assert sum(int(b.plan(i).ncoords[-1]) for i in range(b.size)) == info["total_trials"]
 
 
+def test_batch_of_long_periods_matches_single_series():
+    """Periods of many chunks (few bins of each in a chunk): the grouped launch takes its wide
+    blocks, of 16 to 64 frequencies, beside short-period series."""
+    from loki_amd import libculoki, libloki
+
+    rng = np.random.default_rng(17)
+    lims = [(16, 0.5, 2.0), (32, 0.4, 1.1), (64, 0.5, 1.9), (128, 0.35, 1.2), (64, 9.0, 11.0),
+            (8, 0.6, 2.4)]
+    cfgs = [libloki.configs.PulsarSearchConfig(
+        nsamps=2**18, tsamp=TSAMP, nbins=nb, eta=1.0, param_limits=np.array([[lo, hi]]),
+        use_fourier=False, bseg_brute=2**13) for nb, lo, hi in lims]
+    b = libculoki.ffa.FFABatchCUDA(cfgs, widths=WIDTHS)
+    series = [(rng.standard_normal(2**18, dtype=np.float32),
+               (0.5 + rng.random(2**18)).astype(np.float32)) for _ in cfgs]
+    for i, (e, v) in enumerate(series):
+        b.set_input(i, e, v)
+    b.execute()
+    for i, (e, v) in enumerate(series):
+        single, _ = libculoki.ffa.compute_ffa_scores_cuda(e, v, cfgs[i], widths=b.widths(i))
+        np.testing.assert_array_equal(b.scores(i), single)
+
+
 def test_batch_graph_replays_and_schedules():
     import torch
 

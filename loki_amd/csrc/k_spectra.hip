@@ -257,6 +257,7 @@ k_spectra_fold(SpecFoldArgs a) {
         first[o] = spec_position((ft - floor(ft)) * static_cast<double>(hm[o]), a.m, s, conj[o]);
         spec_weights(s, w[o]);
     }
+    const auto* sums    = reinterpret_cast<const double*>(sp + (npt - 1));  // of the staged chunk
     const uint64_t seg1 = min(seg0 + a.segs_per_block, static_cast<uint64_t>(a.nseg));
     for (uint64_t seg = seg0; seg < seg1; ++seg) {
         float4 acc[OUTS];
@@ -271,9 +272,10 @@ k_spectra_fold(SpecFoldArgs a) {
                 sp[i] = src[i];
             }
             __syncthreads();
-            if (threadIdx.x < 2) {
-                const double x     = reinterpret_cast<const double*>(sp + (npt - 1))[threadIdx.x];
-                s_dc[threadIdx.x] = c == 0 ? x : s_dc[threadIdx.x] + x;
+            if constexpr (TURN) {
+                if (a.nchunk > 1 && threadIdx.x < 2) {
+                    s_dc[threadIdx.x] = c == 0 ? sums[threadIdx.x] : s_dc[threadIdx.x] + sums[threadIdx.x];
+                }
             }
 #pragma unroll
             for (int o = 0; o < OUTS; ++o) {
@@ -292,19 +294,29 @@ k_spectra_fold(SpecFoldArgs a) {
                     acc[o].y += v.y;
                     acc[o].z += v.z;
                     acc[o].w += v.w;
-                } else {
-                    acc[o] = v;
+                } else {  // the only chunk
+                    acc[o] = hm[o] == 0 ? make_float4(static_cast<float>(sums[0]), 0.0F,
+                                                      static_cast<float>(sums[1]), 0.0F)
+                                        : v;
                 }
             }
         }
-        __syncthreads();  // s_dc is complete
-        const auto dc_e = static_cast<float>(s_dc[0]);
-        const auto dc_v = static_cast<float>(s_dc[1]);
+        if constexpr (TURN) {
+            const double* dc = sums;  // the only chunk's
+            if (a.nchunk > 1) {
+                __syncthreads();  // s_dc is complete
+                dc = s_dc;
+            }
+#pragma unroll
+            for (int o = 0; o < OUTS; ++o) {
+                if (hm[o] == 0) {
+                    acc[o] = make_float4(static_cast<float>(dc[0]), 0.0F,
+                                         static_cast<float>(dc[1]), 0.0F);
+                }
+            }
+        }
 #pragma unroll
         for (int o = 0; o < OUTS; ++o) {
-            if (hm[o] == 0) {
-                acc[o] = make_float4(dc_e, 0.0F, dc_v, 0.0F);
-            }
             if (valid[o]) {
                 float2* row = a.fold + ((seg * a.nfreqs + fi[o]) * 2) * a.nbf + hm[o];
                 row[0]      = make_float2(acc[o].x, acc[o].y);

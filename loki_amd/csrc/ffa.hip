@@ -341,7 +341,7 @@ void FFAExecutor::init_level(const float* ts_e, const float* ts_v, void* out, vo
         const auto seglen  = static_cast<uint32_t>(m_plan.segment_lens()[0]);
         const auto nfreqs  = static_cast<uint32_t>(m_plan.param_counts()[0].back());
         const auto nb      = static_cast<uint32_t>(nbins);
-        if (!m_dft_split && kern::spectra_fold_better(nseg, seglen, nfreqs, false)) {
+        if (!m_dft_split && kern::spectra_fold_better(nseg, seglen, nfreqs, nb, false)) {
             // The spectra go into the partner buffer (buffer_size elements), free until
             // the first merge.  Only a plan whose levels are smaller than they are (few
             // frequencies of long segments) keeps a buffer for them.
@@ -841,7 +841,7 @@ void brute_fold_fourier_device(const float* ts_e, const float* ts_v, SizeType ns
     const auto nfreqs  = static_cast<uint32_t>(freqs.size());
     const auto nb      = static_cast<uint32_t>(nbins);
     const SizeType ns  = nsamps / segment_len;
-    const bool spectra = kern::spectra_fold_better(ns, seglen, nfreqs, true);
+    const bool spectra = kern::spectra_fold_better(ns, seglen, nfreqs, nb, true);
     // one allocation: the spectra (16-byte aligned), then the frequencies
     const SizeType spec_bytes =
         spectra ? kern::spectra_bytes(ns, seglen, kern::kMaxSpectraOneOff) : 0;

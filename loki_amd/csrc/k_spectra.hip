@@ -395,25 +395,50 @@ void chunk_spectra(const float* ts_e, const float* ts_v, uint64_t nseg, uint64_t
     }
 }
 
+namespace {
+
+/// Time the spectra save over the matrix cores, in us, without their fixed costs.
+/// Fitted to segments of 64 to 256 samples: a matrix-core fold takes 2.0 ps per
+/// (sample, frequency) for its twiddles and 0.15-0.17 ps per harmonic beyond (the
+/// first 18 share a tile with their neighbours up to 33), 0.7 of it from 128
+/// samples; the FFTs 7 ns per chunk (of c samples, padding included) and 6 ps per
+/// sample (2^23 samples: 0.94, 0.51, 0.29 ms for segments of 64, 128 and 256).
+double spectra_gain_us(uint64_t nseg, uint32_t seglen, uint32_t nfreqs, uint32_t nbf) {
+    const auto sh   = spectra_shape(seglen);
+    const double n  = static_cast<double>(nseg) * seglen;
+    const double c  = sh.m / 2.0;
+    const double pad = c * static_cast<double>(sh.nchunk) / seglen;
+    const double mc = (2.0 + 0.17 * std::min(nbf, 18U) + 0.146 * (nbf > 33 ? nbf - 33.0 : 0.0)) *
+                      (seglen < 128 ? 1.0 : 0.7);
+    return 1e-6 * n * (mc * nfreqs - (7000.0 / c + 6.0) * pad);
+}
+
+}  // namespace
+
 // The spectra cost the same for any number of frequencies, the matrix cores 2 K
-// per value.  Level 0 of a plan, matrix cores against spectra, nbins 16 / 64, us:
-//   2^17 samples, segments of 64:   48 frequencies 28 / 39 against 35 / 38,
-//                                   96 frequencies 47 / 61 against 35 / 53
-//   2^17 samples, segments of 128:  48 frequencies 35 / 38 against 23 / 26
-//   2^23 samples, segments of 128:  32 frequencies 742 / 1026 (spectra about 500),
-//                                   48 frequencies 1076 / 1485 against 546 / 757
-//   2^23 samples, segments of 2048: 48 frequencies 446 / 724 against 148 / 180
-//   2^23 samples, segments of 8192: 2 frequencies 1672 / 873 against 145 / 143
-//                                   (the matrix cores have too few rows)
-// A one-off call allocates the spectra, about 25 us more: 2^17 samples, segments
-// of 128, 48 frequencies 47 / 48 against 63 / 69, 256 frequencies 85 / 129 against
-// 81 / 109; segments of 256, 64 frequencies 69 / 52 against 59 / 67.
-bool spectra_fold_better(uint64_t nseg, uint32_t seglen, uint32_t nfreqs, bool one_off) {
-    uint64_t least = seglen >= 4096 ? 1 : (seglen >= 128 ? 48 : 96);
-    if (one_off && seglen <= 256) {
-        least = std::max<uint64_t>({least, 64, (1ULL << 25) / (std::max<uint64_t>(nseg, 1) * seglen)});
+// per value.  Level 0 of a plan, matrix cores against spectra, us:
+//   2^17 samples, segments of 64: 48 frequencies, 16 bins 28 / 35; 64 frequencies,
+//     64 bins 46 / 53; 96 frequencies, 4 bins 41 / 33, 64 bins 61 / 53
+//   2^23 samples, segments of 64: 48 frequencies, 16 bins 1425 / 1003
+//   2^17 samples, segments of 128: 48 frequencies, 16 bins 35 / 23, 64 bins 38 / 26
+//   2^23 samples, segments of 128: 32 frequencies, 16 bins 742 (spectra about 500)
+//   2^23 samples, segments of 2048: 48 frequencies, 16 bins 446 / 148
+//   2^23 samples, segments of 8192: 2 frequencies, 16 bins 1672 / 145 (the matrix
+//     cores have too few rows)
+// A one-off call allocates the spectra, 25 us and more:
+//   2^17 samples, segments of 128: 64 frequencies, 64 bins 50 / 81, 48, 256 bins 120 / 99
+//   2^20 samples, segments of 128: 48 frequencies, 16 bins 117 / 131, 64 bins 184 / 143
+//   2^17 samples, segments of 256: 64 frequencies, 64 bins 52 / 67, 96 70 / 68
+bool spectra_fold_better(uint64_t nseg, uint32_t seglen, uint32_t nfreqs, uint32_t nbins,
+                         bool one_off) {
+    if (seglen < 64 || (nfreqs < 48 && seglen < 4096)) {
+        return false;
     }
-    return seglen >= 64 && nfreqs >= least;
+    if (seglen > 256 || (!one_off && (seglen >= 128 || nfreqs >= 96))) {
+        return true;
+    }
+    const double least = !one_off ? 40.0 : (seglen <= 128 ? 65.0 : 40.0);
+    return spectra_gain_us(nseg, seglen, nfreqs, nbins / 2 + 1) >= least;
 }
 
 void brute_fold_spectra(const float* ts_e, const float* ts_v, uint64_t nseg, uint32_t seglen,

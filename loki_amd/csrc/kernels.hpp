@@ -161,7 +161,8 @@ void chunk_spectra(const float* ts_e, const float* ts_v, uint64_t nseg, uint64_t
 
 /// Whether brute_fold_spectra is the faster Fourier brute fold; one_off: the
 /// workspace is allocated for the call.
-bool spectra_fold_better(uint64_t nseg, uint32_t seglen, uint32_t nfreqs, bool one_off);
+bool spectra_fold_better(uint64_t nseg, uint32_t seglen, uint32_t nfreqs, uint32_t nbins,
+                         bool one_off);
 /// The Fourier brute fold interpolated from chunk spectra (FP64 FFTs, FP32
 /// values and weights): the same sums as brute_fold_fourier.  spec: spec_bytes of
 /// workspace, 16-byte aligned, at least one segment's spectra; the segments

@@ -23,12 +23,12 @@ U = 2.0**-24
 
 
 @pytest.mark.parametrize(("seglen", "nseg", "nbins", "nfreqs", "t_ref"), [
-    # the smallest chunks, where a one-off fold needs 2^25 (sample, frequency) pairs for them
+    # the smallest chunks, which a one-off fold takes where there is enough work
     (64, 5500, 16, 96, 0.0),
     (65, 5400, 16, 97, 65 * TSAMP / 2),
     (100, 3500, 50, 99, 0.0021),
-    (256, 2050, 2, 64, 0.0),
-    # fewer pairs: the matrix cores, the same bound
+    (256, 2600, 2, 64, 0.0),
+    # less work: the matrix cores, the same bound
     (64, 5, 16, 48, 0.0),
     (65, 3, 64, 57, 65 * TSAMP / 2),    # zero-padded to 128, centre not at t_ref
     (100, 7, 50, 63, 0.0021),

@@ -559,10 +559,10 @@ def run_batch(args, wl) -> int:
             "unit": "TB/s (LDS)",
             "frac": lds_bytes / (ms_per_step * 1e-3) / 1e12 / LDS_PEAK_TBPS, "traffic": None,
             "lds_bytes_per_step": lds_bytes, "sample_freq_pairs": pairs,
-            "note": "8 LDS bytes per (sample, frequency) pair of the brute fold, which takes 95 % "
+            "note": "8 LDS bytes per (sample, frequency) pair of the brute fold, which takes 93 % "
                     "of the step (profiles/batched_uneven_kernel_trace.md; its SQ counters in "
                     "profiles/batched_uneven_brute_fold_sq_counters.md), over the whole step's "
-                    "time, so the fold's own fraction is about 5 % higher; LDS peak 128 B per "
+                    "time, so the fold's own fraction is about 7 % higher; LDS peak 128 B per "
                     "clock per CU",
             "hbm": {"alg_bytes_per_step": alg,
                     "achieved_GBps": alg / (ms_per_step * 1e-3) / 1e9,

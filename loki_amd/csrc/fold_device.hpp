@@ -182,12 +182,13 @@ __device__ __forceinline__ uint32_t run_bound(int64_t u, uint32_t n, double tsam
 // list's.  The next chunk is on its way into registers, and its units are
 // counted by the last wave, while the units of this one are added.
 //
-// VALU and LDS are about equally busy (24 series of 2^18 to 2^21 samples,
-// 1.3e10 (sample, frequency) pairs, 3.9 ms: 9.3 lane-instructions per pair, two
-// of them the adds, and 2.8 ms of LDS cycles, 43 % of them the runs' bank
-// conflicts).  1024 pairs per block leave five blocks on a CU (26 KB of LDS, 86
-// registers); 4096 pairs (three blocks), every boundary by run_bound and the
-// staging unhidden took 5.3 ms.  Chunks of 4096 samples keep more lanes busy
+// VALU and LDS bound it together (256 series of 2^18 to 2^22 samples, 2.6e11
+// (sample, frequency) pairs, 59 ms: 5.8 lane-instructions per pair, two of them
+// the adds, 39 ms of single-issue VALU, and 25 ms a CU of bank conflicts between
+// the lanes' runs).  1024 pairs per block leave five blocks on a CU (26 KB of LDS,
+// 86 registers); 24 series of 2^18 to 2^21 samples, 1.3e10 pairs, take 4.0 ms, and
+// took 5.3 ms with 4096 pairs (three blocks), every boundary by run_bound and the
+// staging unhidden.  Chunks of 4096 samples keep more lanes busy
 // where a launch is too small to fill the chip (2^20 samples, 403 frequencies,
 // 0.5-2 Hz: 0.18 against 0.20 ms, 0.49 ms before; 2^17 samples 0.03 against 0.21
 // ms before); they hold three blocks of 64 bins on a CU (43 KB; four by their 102

@@ -58,7 +58,8 @@ k_chunk_spectra(const float* __restrict__ ts_e, const float* __restrict__ ts_v, 
     const uint64_t k0  = (q % nchunk) * (2 * C);
     const uint32_t len = static_cast<uint32_t>(min(static_cast<uint64_t>(2 * C), seglen - k0));
     const int tid      = static_cast<int>(threadIdx.x);
-    if (users.theta != nullptr) {  // nothing to do if no candidate reads the spectra
+    // nothing to do if no candidate reads the spectra; mostly the first one does
+    if (users.theta != nullptr && !spectral_ok(users.theta, users)) {
         bool any = false;
         for (uint32_t c = threadIdx.x; c < users.ncand && !any; c += T) {
             any = spectral_ok(users.theta + 3 * static_cast<uint64_t>(c), users);
